@@ -33,8 +33,13 @@
  * Calls are stateless and reentrant.  On failure a call returns a nonzero
  * rwkv7m_status and rwkv7m_last_error() describes it (thread-local).
  * Supported head sizes N: 1, 2, 4, 8, 16, 32, 64, 128.  The MFMA chunked
- * kernels serve bf16 with N == 64; every other case runs the sequential
- * kernels, with identical results to the tolerance of the contract.
+ * kernels serve bf16 with N == 64; fp32 with N == 16, 32, 64 or 128 and bf16
+ * with N == 16, 32 or 128 run chunked fp32 kernels from a few dozen tokens
+ * on, whose workspace (at most about 200 MB, more only where a few dozen
+ * chunks of the call's heads need it) comes from a stream-ordered pool;
+ * every other case, and a call whose workspace does not fit, runs the
+ * sequential kernels, with identical results to the tolerance of the
+ * contract.
  */
 #ifndef RWKV7M_WKV_H
 #define RWKV7M_WKV_H
@@ -118,7 +123,9 @@ void rwkv7m_debug_set_forward_segments(int workgroups_per_head);
  * launched: "wave_forward" (MFMA chunked forward), "decode" (single-token
  * kernel), "seq_forward", "wave_backward" (MFMA chunked backward, with the
  * exact sequential pass for any head outside the factored form's range),
- * "seq_backward", or "" (nothing launched).  A diagnostic for tests that
+ * "seq_backward", "f32_forward" and "f32_backward" (chunked fp32 kernels,
+ * with the sequential ones for any head outside their range), or "" (nothing
+ * launched).  A diagnostic for tests that
  * must prove which kernel served a request; no counterpart in the
  * reference.
  */
@@ -152,8 +159,9 @@ int rwkv7m_wkv7_forward(int dtype, int64_t T, int64_t B, int64_t H, int64_t N,
  * needs.  Replaces WKVFFIBackend.forward_with_aux (wkv_ffi.py:33; called at
  * wkv.py:174) and the reference's fwd+aux kernel (wkv_pallas_gpu.py:66-120,
  * :303-375).  checkpoint_interval = 0 selects the library default; the
- * MFMA path serves bf16, N = 64 and an interval of 16, 32 or 64; other
- * intervals run the sequential kernels.
+ * MFMA path serves bf16, N = 64 and an interval of 16, 32 or 64, the chunked
+ * fp32 path multiples of 16 up to 1024 (their backward: 16); other intervals
+ * run the sequential kernels.
  * checkpoints: [rwkv7m_wkv7_checkpoint_count(T, ci)][B][H][N][N] of
  * rwkv7m_wkv7_checkpoint_dtype(dtype, N, ci).
  */

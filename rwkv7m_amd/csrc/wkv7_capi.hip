@@ -177,6 +177,29 @@ bool use_chunked(int dtype, int64_t N, int64_t ci, int64_t T,
     return all_aligned16(ptrs);
 }
 
+// The chunked fp32 kernels serve fp32 vectors with N = 16, 32, 64 or 128 and
+// bf16 ones with N = 16, 32 or 128, 16-byte aligned buffers, chunks whose
+// byte span stays below 2^31 and checkpoint intervals of whole chunks
+// (multiples of 16 up to 1024, which a time segment holds whole; 16
+// backward), from f32_min_tokens on: below that their three to five launches take longer than a sequential kernel's few tokens.
+// Measured as replayed graphs, 4 and 96 heads, chunked against sequential
+// (us): forward N = 64 T 64 29 / 22 and 31 / 23, T 128 36 / 41 and 43 / 43;
+// N = 32 T 192 34 / 38 and 39 / 39; N = 16 T 256 34 / 45 and 38 / 46; N = 128
+// T 64 41 / 49 and 53 / 52.  Backward N = 64 T 32 34 / 51 and 37 / 53; N = 16
+// T 32 28 / 22 and 29 / 22, T 48 28 / 31 and 30 / 31.
+int64_t f32_min_tokens(bool backward, int64_t N) {
+    if (backward) return N == 16 ? 48 : 32;
+    return N == 128 ? 64 : N == 64 ? 128 : N == 32 ? 192 : 256;
+}
+bool use_f32_chunks(int dtype, int64_t N, int64_t T, int64_t BH,
+                    int64_t token_stride, bool backward,
+                    std::initializer_list<const void*> ptrs) {
+    if (N != 16 && N != 32 && N != 64 && N != 128) return false;
+    if (dtype == RWKV7M_DTYPE_BF16 && N == 64) return false;
+    if (token_stride * 64 >= (int64_t(1) << 31)) return false;
+    return T >= f32_min_tokens(backward, N) && BH <= (int64_t(1) << 22) && all_aligned16(ptrs);
+}
+
 int forward_impl(const char* fn, int dtype, int64_t T, int64_t B, int64_t H,
                  int64_t N, const void* r, const void* w, const void* k,
                  const void* v, const void* a, const void* b,
@@ -246,6 +269,16 @@ int forward_impl(const char* fn, int dtype, int64_t T, int64_t B, int64_t H,
         all_aligned16({r, w, k, v, a, b, y, s0, s_t})) {
         g_last_path = "decode";
         return hip_status("decode launch", rwkv7m::launch_decode(p, stream));
+    }
+    if (use_f32_chunks(dtype, N, T, B * H, lay.ts, false,
+                       {r, w, k, v, a, b, y, s0, s_t, ckpt}) &&
+        (!ckpt || (ci % 16 == 0 && ci <= 1024))) {
+        const hipError_t e = rwkv7m::launch_f32_forward(p, stream);
+        if (e != hipErrorOutOfMemory) {
+            g_last_path = "f32_forward";
+            return hip_status("fp32 chunked forward launch", e);
+        }
+        (void)hipGetLastError();  // no room for the workspace
     }
     g_last_path = "seq_forward";
     return hip_status("sequential forward launch",
@@ -383,6 +416,17 @@ int backward_impl(const char* fn, int dtype, int64_t T, int64_t B, int64_t H,
         g_last_path = "wave_backward";
         return hip_status("exact pass launch",
                           rwkv7m::launch_seq_backward(p, s));
+    }
+    if (ci == 16 &&
+        use_f32_chunks(dtype, N, T, B * H, lay.ts, true,
+                       {r, w, k, v, neg_kk, kka, dy, ds_t, checkpoints, dr, dw,
+                        dk, dv, dneg_kk, dkka, ds0, add_dr, add_dk, add_dv})) {
+        const hipError_t e = rwkv7m::launch_f32_backward(p, s);
+        if (e != hipErrorOutOfMemory) {
+            g_last_path = "f32_backward";
+            return hip_status("fp32 chunked backward launch", e);
+        }
+        (void)hipGetLastError();  // no room for the workspace
     }
     g_last_path = "seq_backward";
     return hip_status("sequential backward launch",

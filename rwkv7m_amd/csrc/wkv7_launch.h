@@ -36,6 +36,9 @@ struct SeqFwdArgs {
     void* ckpt;           // nullptr: no checkpoints
     bool ckpt_bf16;       // checkpoint element type: bf16 (else fp32)
     int64_t ci;           // checkpoint interval (when ckpt != nullptr)
+    // nullptr, or [nflag][B * H]: only the heads with a nonzero entry
+    const int* flags;
+    int64_t nflag;
 };
 
 struct SeqBwdArgs {
@@ -55,6 +58,13 @@ struct SeqBwdArgs {
     // nullptr, or cotangents (vector layout and dtype) added to dr, dk, dv
     // in fp32 before they are rounded and stored
     const void *add_dr, *add_dk, *add_dv;
+    // nullptr, or [nflag][B * H]: only the heads with a nonzero entry.
+    // Row-split heads (N = 128) then keep their column sums' shares at
+    // `part`, room for 2 * T * B * H * 5 * N floats, and their marks are
+    // gathered in flags' first row.
+    int* flags;
+    int64_t nflag;
+    float* part;
 };
 
 // Bit pattern (a NaN no arithmetic produces) that the wave backward leaves in
@@ -107,6 +117,18 @@ hipError_t launch_wave_backward(const WaveBwdArgs& p, hipStream_t stream);
 void set_backward_segments(int k);
 
 hipError_t launch_seq_forward(const SeqFwdArgs& p, hipStream_t stream);
+
+// Chunked fp32 kernels (wkv7_f32.hip) for the calls the sequential ones
+// served: N in {16, 32, 64, 128} (64 with fp32 vectors only), 16-byte aligned
+// buffers, fp32 checkpoints every multiple of 16 tokens (backward: every
+// 16).  hipErrorOutOfMemory, with nothing launched, where their workspace
+// does not fit.
+hipError_t launch_f32_forward(const SeqFwdArgs& p, hipStream_t stream);
+hipError_t launch_f32_backward(const SeqBwdArgs& p, hipStream_t stream);
+
+// Device memory from a stream-ordered pool per device, freed with
+// hipFreeAsync.
+hipError_t pool_alloc(float** out, size_t bytes, hipStream_t stream);
 
 // Fused time-mix producers and consumer (wkv7_timemix.hip).  Activations are
 // [rows][C] of the launch dtype; parameters fp32 [C]; N in {8, ..., 128}.

@@ -4,8 +4,9 @@
 // Each state row i is owned by G consecutive lanes, each holding C = N / G
 // contiguous columns in VGPRs, so the row-local parts of the recurrence
 // (sa = S a, y = S r, the rank-2 update) need only a G-lane butterfly.
-// Token vectors are staged through LDS in blocks.  These kernels carry the
-// fp32 path, every head size, and the exact fallback of the chunked path.
+// Token vectors are staged through LDS in blocks.  These kernels serve
+// what the chunked paths do not (N <= 8, short sequences, other checkpoint
+// intervals, misaligned buffers) and the heads outside their range.
 //
 // Math (reference src/rwkv7m/model/rwkv_core.py:54-86):
 //   d = exp(-exp(w));  sa = S a;  S = S diag(d) + sa b^T + v k^T;  y = S r
@@ -75,6 +76,17 @@ __device__ __forceinline__ float raw_to_f(bf16_t x) {
     return __uint_as_float(uint32_t(x) << 16);
 }
 
+// Whether head bh has a nonzero entry in flags[nflag][BH] (or there are no
+// flags).
+__device__ __forceinline__ bool wanted(const int* flags, int64_t nflag,
+                                       int64_t BH, int64_t bh) {
+    if (!flags) return true;
+    int f = 0;
+    for (int64_t i = threadIdx.x % 64; i < nflag; i += 64)
+        f |= flags[i * BH + bh];
+    return __any(f);
+}
+
 // Forward.  ckpt == nullptr: no aux.  s_t may alias s0.  CT is the
 // checkpoint element type (float or bf16_t).
 template <int N, typename VT, typename CT>
@@ -84,7 +96,8 @@ wkv7_seq_fwd_kernel(int64_t T, int64_t BH, VecLayout lay,
                     const VT* __restrict__ w, const VT* __restrict__ k,
                     const VT* __restrict__ v, const VT* __restrict__ a,
                     const VT* __restrict__ b, const float* s0, VT* y,
-                    float* s_t, CT* ckpt, int64_t ci) {
+                    float* s_t, CT* ckpt, int64_t ci,
+                    const int* __restrict__ flags, int64_t nflag) {
     using Sh = SeqShape<N>;
     constexpr int G = Sh::G, C = Sh::C, TB = Sh::TB, TH = Sh::THREADS;
     constexpr int64_t NN = int64_t(N) * N;
@@ -93,6 +106,7 @@ wkv7_seq_fwd_kernel(int64_t T, int64_t BH, VecLayout lay,
 
     constexpr int NR = Sh::NR;
     const int64_t bh = blockIdx.x / Sh::RS;
+    if (!wanted(flags, nflag, BH, bh)) return;
     const int split = int(blockIdx.x % Sh::RS);
     const int tid = threadIdx.x;
     const int row = split * NR + tid / G, col0 = (tid % G) * C;
@@ -318,7 +332,7 @@ wkv7_seq_bwd_kernel(int64_t T, int64_t BH, VecLayout lay,
                     const VT* __restrict__ add_dk,
                     const VT* __restrict__ add_dv, int64_t c_lo,
                     int64_t c_hi, float* __restrict__ part, int64_t pt0,
-                    int64_t pT) {
+                    int64_t pT, int* flags, int64_t nflag) {
     using Sh = SeqShape<N>;
     constexpr int G = Sh::G, C = Sh::C, SUB = Sh::SUB, TH = Sh::THREADS;
     constexpr int WL = Sh::WAVE_LANES, NW = Sh::NWAVES;
@@ -339,6 +353,9 @@ wkv7_seq_bwd_kernel(int64_t T, int64_t BH, VecLayout lay,
     if (marked_only &&
         __float_as_uint(ds0[bh * NN]) != kExactPassMark)
         return;
+    if (!wanted(flags, nflag, BH, bh)) return;
+    // (the sum kernel looks at the first row of flags only)
+    if (Sh::RS > 1 && flags && threadIdx.x == 0) flags[bh] = 1;
     const int tid = threadIdx.x;
     const int row = split * NR + tid / G, col0 = (tid % G) * C;
     const int wave = tid / 64, lane = tid % 64;
@@ -585,7 +602,7 @@ wkv7_seq_colsum_kernel(int64_t nt, int64_t t0, int64_t BH, VecLayout lay,
                        const VT* __restrict__ w,
                        const VT* __restrict__ add_dr,
                        const VT* __restrict__ add_dk, VT* dr, VT* dw, VT* db,
-                       VT* dk, VT* da) {
+                       VT* dk, VT* da, const int* __restrict__ flags) {
     constexpr int RS = SeqShape<N>::RS;
     const int64_t per = BH * 5 * N;  // values per token
     const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -593,6 +610,7 @@ wkv7_seq_colsum_kernel(int64_t nt, int64_t t0, int64_t BH, VecLayout lay,
     const int64_t tl = e / per;
     const int64_t rem = e - tl * per;
     const int64_t bh = rem / (5 * N);
+    if (flags && !flags[bh]) return;
     const int qj = int(rem - bh * (5 * N));
     const int q = qj / N, j = qj - q * N;
     float acc = 0.f;
@@ -607,42 +625,6 @@ wkv7_seq_colsum_kernel(int64_t nt, int64_t t0, int64_t BH, VecLayout lay,
     if (q == 3 && add_dk) acc += load_f(add_dk + off);
     VT* gout[5] = {dr, dw, db, dk, da};
     store_f(gout[q] + off, acc);
-}
-
-// Device memory for the row-split backward's partial column sums: a
-// stream-ordered pool per device that keeps what it has reserved (so
-// repeated calls reuse it instead of mapping new memory each time).
-constexpr int kPoolDevices = 64;
-std::mutex g_pool_mu;
-hipMemPool_t g_pool[kPoolDevices];
-
-hipError_t part_alloc(float** out, size_t bytes, hipStream_t stream) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kPoolDevices) return hipErrorInvalidDevice;
-    {
-        std::lock_guard<std::mutex> lock(g_pool_mu);
-        if (g_pool[dev] == nullptr) {
-            hipMemPoolProps props{};
-            props.allocType = hipMemAllocationTypePinned;
-            props.location.type = hipMemLocationTypeDevice;
-            props.location.id = dev;
-            hipMemPool_t pool = nullptr;
-            e = hipMemPoolCreate(&pool, &props);
-            if (e != hipSuccess) return e;
-            uint64_t keep = UINT64_MAX;
-            e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold,
-                                       &keep);
-            if (e != hipSuccess) {
-                hipMemPoolDestroy(pool);
-                return e;
-            }
-            g_pool[dev] = pool;
-        }
-    }
-    return hipMallocFromPoolAsync(reinterpret_cast<void**>(out), bytes,
-                                  g_pool[dev], stream);
 }
 
 // Partial column sums held at once by a row-split backward (bytes): the
@@ -662,7 +644,7 @@ hipError_t launch_fwd_nc(const SeqFwdArgs& p, hipStream_t stream) {
                        static_cast<const VT*>(p.a),
                        static_cast<const VT*>(p.b), p.s0,
                        static_cast<VT*>(p.y), p.s_t,
-                       static_cast<CT*>(p.ckpt), p.ci);
+                       static_cast<CT*>(p.ckpt), p.ci, p.flags, p.nflag);
     return hipGetLastError();
 }
 
@@ -695,7 +677,7 @@ hipError_t launch_bwd_seg(const SeqBwdArgs& p, const float* ds_in,
                        static_cast<const VT*>(p.add_dr),
                        static_cast<const VT*>(p.add_dk),
                        static_cast<const VT*>(p.add_dv), c_lo, c_hi, part,
-                       pt0, pT);
+                       pt0, pT, p.flags, p.nflag);
     return hipGetLastError();
 }
 
@@ -714,10 +696,12 @@ hipError_t launch_bwd_nc(const SeqBwdArgs& p, hipStream_t stream) {
         const int64_t tok_bytes = int64_t(RS) * BH * 5 * N * 4;
         int64_t seg = kPartBytes / (tok_bytes * p.ci);
         if (seg < 1) seg = 1;
-        if (seg > nint) seg = nint;
+        if (seg > nint || p.part) seg = nint;
         const int64_t seg_tok = seg * p.ci < p.T ? seg * p.ci : p.T;
-        float* part = nullptr;
-        hipError_t e = part_alloc(&part, size_t(seg_tok * tok_bytes), stream);
+        float* part = p.part;
+        hipError_t e = hipSuccess;
+        if (!part)
+            e = pool_alloc(&part, size_t(seg_tok * tok_bytes), stream);
         if (e != hipSuccess) return e;
         // segments of `seg` intervals, the last first; dS passes from one to
         // the next through dS0 (each lane reads its own values before it
@@ -739,10 +723,11 @@ hipError_t launch_bwd_nc(const SeqBwdArgs& p, hipStream_t stream) {
                                static_cast<const VT*>(p.add_dk),
                                static_cast<VT*>(p.dr), static_cast<VT*>(p.dw),
                                static_cast<VT*>(p.db), static_cast<VT*>(p.dk),
-                               static_cast<VT*>(p.da));
+                               static_cast<VT*>(p.da), p.flags);
             e = hipGetLastError();
             c_hi = c_lo;
         }
+        if (p.part) return e;
         const hipError_t f = hipFreeAsync(part, stream);
         return e != hipSuccess ? e : f;
     }
@@ -785,6 +770,44 @@ hipError_t dispatch_bwd(const SeqBwdArgs& p, hipStream_t s) {
 }
 
 }  // namespace
+
+namespace {
+// The pools keep up to kPoolKeep bytes reserved when nothing is in use, so
+// that repeated calls reuse them instead of mapping new memory each time.
+constexpr uint64_t kPoolKeep = uint64_t(512) << 20;
+constexpr int kPoolDevices = 64;
+std::mutex g_pool_mu;
+hipMemPool_t g_pool[kPoolDevices];
+}  // namespace
+
+hipError_t pool_alloc(float** out, size_t bytes, hipStream_t stream) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kPoolDevices) return hipErrorInvalidDevice;
+    {
+        std::lock_guard<std::mutex> lock(g_pool_mu);
+        if (g_pool[dev] == nullptr) {
+            hipMemPoolProps props{};
+            props.allocType = hipMemAllocationTypePinned;
+            props.location.type = hipMemLocationTypeDevice;
+            props.location.id = dev;
+            hipMemPool_t pool = nullptr;
+            e = hipMemPoolCreate(&pool, &props);
+            if (e != hipSuccess) return e;
+            uint64_t keep = kPoolKeep;
+            e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold,
+                                       &keep);
+            if (e != hipSuccess) {
+                (void)hipMemPoolDestroy(pool);
+                return e;
+            }
+            g_pool[dev] = pool;
+        }
+    }
+    return hipMallocFromPoolAsync(reinterpret_cast<void**>(out), bytes,
+                                  g_pool[dev], stream);
+}
 
 hipError_t launch_seq_forward(const SeqFwdArgs& p, hipStream_t stream) {
     return p.bf16 ? dispatch_fwd<bf16_t>(p, stream)

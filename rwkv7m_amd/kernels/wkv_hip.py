@@ -252,8 +252,8 @@ def _layout(layout: str, r: torch.Tensor):
 
 def last_path() -> str:
     """Kernel path of the last successful WKV-7 call on this thread
-    ("wave_forward", "decode", "seq_forward", "wave_backward",
-    "seq_backward" or "")."""
+    ("wave_forward", "decode", "seq_forward", "f32_forward",
+    "wave_backward", "seq_backward", "f32_backward" or "")."""
     return load_library().rwkv7m_wkv7_last_path().decode()
 
 

@@ -1,0 +1,158 @@
+"""The chunked fp32 kernels (wkv7_f32.hip) against the float64 oracle: every
+head size, both vector types and layouts, whole and partial last chunks,
+intervals other than the chunk, absent cotangents, added cotangents, and heads
+whose chunks leave the factored form's range (served by the sequential
+kernels).  Tolerances are the repository's: 1e-4 (fp32) and 2e-2 (bf16) of the
+oracle's largest magnitude; the kernels' own error is 2e-7 (fp32) or the bf16
+rounding of the outputs (4e-3).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from rwkv7m_amd.synthetic import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("r", "w", "k", "v", "neg_kk", "kka")
+GRADS = ("dr", "dw", "dk", "dv", "dneg_kk", "dkka", "ds0")
+TOL = {torch.float32: 1e-4, torch.bfloat16: 2e-2}
+
+
+@pytest.fixture(scope="module")
+def hip(hip_lib):
+    from rwkv7m_amd.kernels import wkv_hip
+    return wkv_hip
+
+
+def _np(t):
+    return t.detach().float().cpu().numpy().astype(np.float64)
+
+
+def _close(name, got, want, tol, tag):
+    err = oracle.normalized_max_error(_np(got), want)
+    assert err <= tol, f"{tag} {name}: {err:.3e} > {tol}"
+
+
+def _dev(inp, layout):
+    t = {n: x.cuda() for n, x in inp.items()}
+    if layout == "bthn":
+        for n in (*NAMES, "dy"):
+            t[n] = t[n].transpose(0, 1).contiguous()
+    return t
+
+
+CASES = [
+    # T, B, H, N, dtype, layout
+    (256, 1, 2, 16, torch.float32, "tbhn"),
+    (273, 2, 1, 16, torch.bfloat16, "bthn"),
+    (192, 1, 3, 32, torch.float32, "bthn"),
+    (207, 1, 2, 32, torch.bfloat16, "tbhn"),
+    (128, 1, 2, 64, torch.float32, "tbhn"),
+    (145, 2, 2, 64, torch.float32, "bthn"),
+    (64, 1, 1, 128, torch.float32, "tbhn"),
+    (97, 1, 3, 128, torch.bfloat16, "bthn"),
+]
+
+
+@pytest.mark.parametrize("T,B,H,N,dtype,layout", CASES)
+def test_matches_oracle(hip, T, B, H, N, dtype, layout):
+    tag = f"T{T} B{B} H{H} N{N} {dtype} {layout}"
+    print("case: chunked fp32", tag, flush=True)
+    inp = make_inputs(T, B, H, N, dtype=dtype, seed=T + N, state_std=0.1,
+                      dstate_std=0.1)
+    host = [_np(inp[n]) for n in NAMES]
+    ey, es, eck = oracle.forward(*host, _np(inp["s0"]),
+                                 checkpoint_interval=16)
+    eg = oracle.backward(*host, _np(inp["s0"]), _np(inp["dy"]),
+                         _np(inp["ds_t"]))
+    if layout == "bthn":
+        ey = ey.swapaxes(0, 1)
+        eg = [g.swapaxes(0, 1) for g in eg[:6]] + [eg[6]]
+    d = _dev(inp, layout)
+    vecs = [d[n] for n in (*NAMES, "s0")]
+    (y, s_t), aux = hip.forward_with_aux(*vecs, layout=layout)
+    assert hip.last_path() == "f32_forward", tag
+    call = dict(layout=layout)
+    grads = hip.backward(*vecs, d["dy"], d["ds_t"], *aux, **call)
+    assert hip.last_path() == "f32_backward", tag
+    y2, s2 = hip.forward(*vecs, layout=layout)
+    again = hip.backward(*vecs, d["dy"], d["ds_t"], *aux, **call)
+    torch.cuda.synchronize()
+    _close("y", y, ey, TOL[dtype], tag)
+    _close("s_t", s_t, es, 1e-4, tag)
+    _close("checkpoints", aux[0], eck, 1e-4, tag)
+    for n, g, e in zip(GRADS, grads, eg):
+        _close(n, g, e, 1e-4 if n == "ds0" else TOL[dtype], tag)
+    assert torch.equal(y, y2) and torch.equal(s_t, s2)
+    assert all(torch.equal(a, b) for a, b in zip(grads, again))
+    # an interval of three chunks: the same kernels, fewer checkpoints
+    (y3, s3), aux3 = hip.forward_with_aux(*vecs, checkpoint_interval=48,
+                                          layout=layout)
+    assert hip.last_path() == "f32_forward"
+    torch.cuda.synchronize()
+    assert torch.equal(y, y3) and torch.equal(s_t, s3)
+    assert torch.equal(aux3[0][:-1], aux[0][:-1:3])
+    assert torch.equal(aux3[0][-1], s_t)
+    # absent cotangents are zeros
+    z = hip.backward(*vecs, torch.zeros_like(d["dy"]), d["ds_t"], *aux, **call)
+    n = hip.backward(*vecs, None, d["ds_t"], *aux, **call)
+    assert all(torch.equal(a, b) for a, b in zip(z, n))
+    if layout == "bthn":  # cotangents of r, k, v from other uses
+        adds = [torch.randn(y.shape, device="cuda").to(dtype) for _ in range(3)]
+        summed = hip.backward(*vecs, d["dy"], d["ds_t"], *aux, layout=layout,
+                              add=adds)
+        assert hip.last_path() == "f32_backward"
+        torch.cuda.synchronize()
+        for i, a in zip((0, 2, 3), adds):
+            _close(f"{GRADS[i]} + added", summed[i], eg[i] + _np(a),
+                   TOL[dtype], tag)
+        for i in (1, 4, 5, 6):
+            assert torch.equal(summed[i], grads[i])
+
+
+@pytest.mark.parametrize("N,dtype", [(64, torch.float32),
+                                     (128, torch.bfloat16)])
+def test_heads_out_of_range_take_the_sequential_kernels(hip, N, dtype):
+    T, H = 150, 3
+    print("case: chunked fp32, heads out of range, N", N, flush=True)
+    inp = make_inputs(T, 1, H, N, dtype=dtype, seed=5, state_std=0.1,
+                      dstate_std=0.1)
+    plain = {n: x.clone() for n, x in inp.items()}
+    inp["w"][40:44, :, 1] = 4.0  # decays of exp(-55) in one chunk of head 1
+    outs = []
+    for x in (plain, inp):
+        d = _dev(x, "tbhn")
+        vecs = [d[n] for n in (*NAMES, "s0")]
+        (y, s_t), aux = hip.forward_with_aux(*vecs)
+        assert hip.last_path() == "f32_forward"
+        g = hip.backward(*vecs, d["dy"], d["ds_t"], *aux)
+        assert hip.last_path() == "f32_backward"
+        outs.append([y, *g[:6], s_t[None], g[6][None]])
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):  # the other heads do not change
+        assert torch.equal(a[:, :, ::2], b[:, :, ::2])
+    host = [_np(inp[n]) for n in NAMES]
+    ey, es = oracle.forward(*host, _np(inp["s0"]))
+    eg = oracle.backward(*host, _np(inp["s0"]), _np(inp["dy"]),
+                         _np(inp["ds_t"]))
+    for n, got, e in zip(("y", *GRADS[:6], "s_t", "ds0"), outs[1],
+                         (ey, *eg[:6], es[None], eg[6][None])):
+        _close(n, got, e, TOL[dtype], f"N{N} strong decay")
+
+
+def test_a_value_out_of_range_does_not_reach_earlier_tokens(hip):
+    print("case: chunked fp32, an infinite v", flush=True)
+    inp = make_inputs(130, 1, 2, 64, dtype=torch.float32, seed=6)
+    inp["v"][70, 0, 0, 3] = float("inf")
+    d = _dev(inp, "tbhn")
+    y, _ = hip.forward(*[d[n] for n in (*NAMES, "s0")])
+    assert hip.last_path() == "f32_forward"
+    torch.cuda.synchronize()
+    assert torch.isfinite(y[:70]).all() and torch.isfinite(y[:, :, 1]).all()
+    rows = torch.arange(64) != 3  # state rows are independent
+    assert torch.isfinite(y[:, 0, 0, rows.cuda()]).all()
