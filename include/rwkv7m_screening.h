@@ -134,6 +134,65 @@ int rwkv7m_screen_write_backward(
     float *d_embed_part, float *d_mu_bm, float *d_kraw, float *dq_w,
     float *d_tau_w, void *stream);
 
+/*
+ * Passes of the module around its GEMMs and recurrences
+ * (nnx_model.py:1015-1160); each dtype argument is the element type of the
+ * tensors named after it, everything else fp32.
+ */
+
+/* Row groups of the partial sums below for `rows` rows (1 .. 256), or -1. */
+int64_t rwkv7m_screen_row_groups(int64_t rows);
+
+/* out = LayerNorm(x) scale + bias over the C columns of each row; mean, rstd
+ * [rows] for the backward. */
+int rwkv7m_screen_norm(int x_dtype, int out_dtype, int64_t rows, int64_t C,
+                       const void *x, const float *scale, const float *bias,
+                       double eps, void *out, float *mean, float *rstd,
+                       void *stream);
+/* dx, and part [row groups][2][C]: summed over the groups, d scale and
+ * d bias. */
+int rwkv7m_screen_norm_backward(int x_dtype, int out_dtype, int64_t rows,
+                                int64_t C, const void *x, const float *scale,
+                                const float *mean, const float *rstd,
+                                const void *dout, void *dx, float *part,
+                                void *stream);
+
+/* out = x / sqrt(sum_n x^2 + eps^2) per row, fp32; and its adjoint. */
+int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void *x,
+                       double eps, float *out, void *stream);
+int rwkv7m_screen_unit_backward(int x_dtype, int64_t rows, int64_t n,
+                                const void *x, double eps, const float *dout,
+                                void *dx, void *stream);
+
+/* h = h_base + lam sigmoid(pre + bias) read; lam one fp32 on the device. */
+int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t rows, int64_t C,
+                           const void *pre, const float *bias,
+                           const float *lam, const void *read,
+                           const void *h_base, void *h, void *stream);
+/* d_pre, d_read, and part [row groups][2][C]: summed over the groups, d bias,
+ * and d lam per column. */
+int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t rows,
+                                    int64_t C, const void *pre,
+                                    const float *bias, const float *lam,
+                                    const void *read, const void *dh,
+                                    void *d_pre, void *d_read, float *part,
+                                    void *stream);
+
+/*
+ * The usage EMA and the statistics from rel, rel_w (NULL: no writes)
+ * [B][T][M], z_norm, u_norm [B][T], upd2 [B][T][M][ndw] and usage0 [B][M].
+ * usage_T [B][M]; stats [10]: mean rel, mean over the steps of the largest
+ * rel, active slots per token, mean rel_w, mean max(rel_w, floor), mean
+ * activity, mean update norm, mean z_norm, mean u_norm, mean over the steps
+ * of the mean EMA.  part: [T][9] floats of scratch.
+ */
+int rwkv7m_screen_stats(int64_t B, int64_t T, int64_t M, int64_t ndw,
+                        const float *rel, const float *rel_w,
+                        const float *z_norm, const float *u_norm,
+                        const float *upd2, const float *usage0, double floor,
+                        double decay, float *part, float *stats,
+                        float *usage_T, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -542,6 +542,24 @@ int sc_dims(const char* fn, int dtype, int64_t B, int64_t T, int64_t M,
     return RWKV7M_OK;
 }
 
+// Rows of the fused passes: their grids hold rows / 4 and C / 64 blocks.
+int sc_rows(const char* fn, int dtype_a, int dtype_b, int64_t rows,
+            int64_t C) {
+    for (int d : {dtype_a, dtype_b})
+        if (d != RWKV7M_DTYPE_F32 && d != RWKV7M_DTYPE_BF16)
+            return fail(RWKV7M_ERR_INVALID_ARGUMENT,
+                        std::string(fn) + ": tensors must be bfloat16 or "
+                                          "float32 (dtype=" +
+                            std::to_string(d) + ")");
+    if (rows < 0 || C < 0)
+        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
+                    std::string(fn) + ": negative dimension");
+    if (rows > (int64_t(1) << 25) || C > (int64_t(1) << 25))
+        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
+                    std::string(fn) + ": sizes too large");
+    return RWKV7M_OK;
+}
+
 int sc_need(const char* fn, std::initializer_list<Named> ptrs) {
     for (const Named& x : ptrs)
         if (x.p == nullptr)
@@ -1111,6 +1129,209 @@ int rwkv7m_screen_slot_scan_backward(
                       rwkv7m::launch_screen_scan(
                           dtype == RWKV7M_DTYPE_BF16, true, A,
                           static_cast<hipStream_t>(stream)));
+}
+
+int64_t rwkv7m_screen_row_groups(int64_t rows) {
+    g_last_error.clear();
+    if (rows < 0) {
+        fail(RWKV7M_ERR_INVALID_ARGUMENT,
+             "rwkv7m_screen_row_groups: rows must be >= 0");
+        return -1;
+    }
+    return rwkv7m::screen_row_groups(rows);
+}
+
+int rwkv7m_screen_norm(int x_dtype, int out_dtype, int64_t rows, int64_t C,
+                       const void* x, const float* scale, const float* bias,
+                       double eps, void* out, float* mean, float* rstd,
+                       void* stream) {
+    const char* fn = "rwkv7m_screen_norm";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, x_dtype, out_dtype, rows, C));
+    if (!(eps >= 0.0))
+        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
+                    std::string(fn) + ": eps must be >= 0");
+    if (rows == 0 || C == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"scale", scale}, {"bias", bias},
+                            {"out", out}, {"mean", mean}, {"rstd", rstd}}));
+    rwkv7m::ScreenNormArgs A{};
+    A.rows = rows;
+    A.C = C;
+    A.eps = float(eps);
+    A.x = x;
+    A.scale = scale;
+    A.bias = bias;
+    A.out = out;
+    A.mean = mean;
+    A.rstd = rstd;
+    return hip_status("screening norm launch",
+                      rwkv7m::launch_screen_norm(
+                          x_dtype == RWKV7M_DTYPE_BF16,
+                          out_dtype == RWKV7M_DTYPE_BF16, false, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_norm_backward(int x_dtype, int out_dtype, int64_t rows,
+                                int64_t C, const void* x, const float* scale,
+                                const float* mean, const float* rstd,
+                                const void* dout, void* dx, float* part,
+                                void* stream) {
+    const char* fn = "rwkv7m_screen_norm_backward";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, x_dtype, out_dtype, rows, C));
+    if (rows == 0 || C == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"scale", scale}, {"mean", mean},
+                            {"rstd", rstd}, {"dout", dout}, {"dx", dx},
+                            {"part", part}}));
+    rwkv7m::ScreenNormArgs A{};
+    A.rows = rows;
+    A.C = C;
+    A.x = x;
+    A.scale = scale;
+    A.mean = const_cast<float*>(mean);
+    A.rstd = const_cast<float*>(rstd);
+    A.dout = dout;
+    A.dx = dx;
+    A.part = part;
+    return hip_status("screening norm backward launch",
+                      rwkv7m::launch_screen_norm(
+                          x_dtype == RWKV7M_DTYPE_BF16,
+                          out_dtype == RWKV7M_DTYPE_BF16, true, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void* x,
+                       double eps, float* out, void* stream) {
+    const char* fn = "rwkv7m_screen_unit";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, x_dtype, x_dtype, rows, n));
+    if (rows == 0 || n == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"out", out}}));
+    rwkv7m::ScreenUnitArgs A{};
+    A.rows = rows;
+    A.n = n;
+    A.eps = float(eps);
+    A.x = x;
+    A.out = out;
+    return hip_status("screening unit norm launch",
+                      rwkv7m::launch_screen_unit(
+                          x_dtype == RWKV7M_DTYPE_BF16, false, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_unit_backward(int x_dtype, int64_t rows, int64_t n,
+                                const void* x, double eps, const float* dout,
+                                void* dx, void* stream) {
+    const char* fn = "rwkv7m_screen_unit_backward";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, x_dtype, x_dtype, rows, n));
+    if (rows == 0 || n == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"dout", dout}, {"dx", dx}}));
+    rwkv7m::ScreenUnitArgs A{};
+    A.rows = rows;
+    A.n = n;
+    A.eps = float(eps);
+    A.x = x;
+    A.dout = dout;
+    A.dx = dx;
+    return hip_status("screening unit norm backward launch",
+                      rwkv7m::launch_screen_unit(
+                          x_dtype == RWKV7M_DTYPE_BF16, true, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t rows, int64_t C,
+                           const void* pre, const float* bias,
+                           const float* lam, const void* read,
+                           const void* h_base, void* h, void* stream) {
+    const char* fn = "rwkv7m_screen_residual";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, pre_dtype, h_dtype, rows, C));
+    if (rows == 0 || C == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"bias", bias}, {"lam", lam},
+                            {"read", read}, {"h_base", h_base}, {"h", h}}));
+    rwkv7m::ScreenResidualArgs A{};
+    A.rows = rows;
+    A.C = C;
+    A.pre = pre;
+    A.bias = bias;
+    A.lam = lam;
+    A.read = read;
+    A.h_base = h_base;
+    A.h = h;
+    return hip_status("screening residual launch",
+                      rwkv7m::launch_screen_residual(
+                          pre_dtype == RWKV7M_DTYPE_BF16,
+                          h_dtype == RWKV7M_DTYPE_BF16, false, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t rows,
+                                    int64_t C, const void* pre,
+                                    const float* bias, const float* lam,
+                                    const void* read, const void* dh,
+                                    void* d_pre, void* d_read, float* part,
+                                    void* stream) {
+    const char* fn = "rwkv7m_screen_residual_backward";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_rows(fn, pre_dtype, h_dtype, rows, C));
+    if (rows == 0 || C == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"bias", bias}, {"lam", lam},
+                            {"read", read}, {"dh", dh}, {"d_pre", d_pre},
+                            {"d_read", d_read}, {"part", part}}));
+    rwkv7m::ScreenResidualArgs A{};
+    A.rows = rows;
+    A.C = C;
+    A.pre = pre;
+    A.bias = bias;
+    A.lam = lam;
+    A.read = read;
+    A.dh = dh;
+    A.d_pre = d_pre;
+    A.d_read = d_read;
+    A.part = part;
+    return hip_status("screening residual backward launch",
+                      rwkv7m::launch_screen_residual(
+                          pre_dtype == RWKV7M_DTYPE_BF16,
+                          h_dtype == RWKV7M_DTYPE_BF16, true, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_stats(int64_t B, int64_t T, int64_t M, int64_t ndw,
+                        const float* rel, const float* rel_w,
+                        const float* z_norm, const float* u_norm,
+                        const float* upd2, const float* usage0, double floor,
+                        double decay, float* part, float* stats,
+                        float* usage_T, void* stream) {
+    const char* fn = "rwkv7m_screen_stats";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_dims(fn, RWKV7M_DTYPE_F32, B, T, M, ndw, 0));
+    if (B == 0 || T == 0 || M == 0)
+        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
+                    std::string(fn) + ": no steps, batch rows or slots");
+    RWKV7M_TRY(sc_need(fn, {{"rel", rel}, {"z_norm", z_norm},
+                            {"u_norm", u_norm}, {"upd2", upd2},
+                            {"usage0", usage0}, {"part", part},
+                            {"stats", stats}, {"usage_T", usage_T}}));
+    rwkv7m::ScreenStatsArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.ndw = ndw;
+    A.rel = rel;
+    A.rel_w = rel_w;
+    A.z_norm = z_norm;
+    A.u_norm = u_norm;
+    A.upd2 = upd2;
+    A.usage0 = usage0;
+    A.floor = float(floor);
+    A.decay = decay;
+    A.part = part;
+    A.stats = stats;
+    A.usage_T = usage_T;
+    return hip_status("screening statistics launch",
+                      rwkv7m::launch_screen_stats(
+                          A, static_cast<hipStream_t>(stream)));
 }
 
 int rwkv7m_screen_read(int dtype, int64_t B, int64_t T, int64_t M,

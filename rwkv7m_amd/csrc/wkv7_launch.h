@@ -233,6 +233,56 @@ hipError_t launch_screen_scan(bool bf16, bool backward,
 hipError_t launch_screen_read(bool bf16, bool backward,
                               const ScreenReadArgs& A, hipStream_t stream);
 
+// The screening module's passes around its GEMMs and recurrences
+// (screen_fused.hip).  part: [screen_row_groups(rows)][2][C] partial sums.
+struct ScreenNormArgs {
+    int64_t rows, C;
+    float eps;
+    const void* x;
+    const float *scale, *bias;
+    void* out;
+    float *mean, *rstd;  // [rows]
+    const void* dout;
+    void* dx;
+    float* part;  // d scale, d bias
+};
+struct ScreenUnitArgs {
+    int64_t rows, n;
+    float eps;
+    const void* x;
+    float* out;
+    const float* dout;
+    void* dx;
+};
+struct ScreenResidualArgs {
+    int64_t rows, C;
+    const void* pre;
+    const float *bias, *lam;
+    const void *read, *h_base;
+    void* h;
+    const void* dh;
+    void *d_pre, *d_read;
+    float* part;  // d bias, and d lam per column
+};
+struct ScreenStatsArgs {
+    int64_t B, T, M, ndw;
+    const float *rel, *rel_w;  // [B][T][M]; rel_w may be 0
+    const float *z_norm, *u_norm, *upd2, *usage0;
+    float floor;
+    double decay;
+    float* part;  // [T][9]
+    float *stats, *usage_T;  // [10], [B][M]
+};
+int64_t screen_row_groups(int64_t rows);
+hipError_t launch_screen_norm(bool x_bf16, bool out_bf16, bool backward,
+                              const ScreenNormArgs& A, hipStream_t stream);
+hipError_t launch_screen_unit(bool bf16, bool backward,
+                              const ScreenUnitArgs& A, hipStream_t stream);
+hipError_t launch_screen_residual(bool pre_bf16, bool h_bf16, bool backward,
+                                  const ScreenResidualArgs& A,
+                                  hipStream_t stream);
+hipError_t launch_screen_stats(const ScreenStatsArgs& A, hipStream_t stream);
+
 int64_t timemix_workspace_floats(int64_t rows, int64_t C);
 hipError_t launch_timemix_inputs(bool bf16, int N, const TmInputsArgs& A,
                                  hipStream_t stream);

@@ -241,3 +241,130 @@ def write_backward(base, slot_term, slot_embed, kw, q_w, tau_w, mu, floor,
           P(_f32(d_slots_T)), P(_f32(d_rel_w)), P(_f32(d_ages_seq)),
           P(_f32(d_ages_T)), *map(P, outs), wkv_hip._stream(dev))
     return tuple(outs)
+
+
+def _parts(rows, C, dev):
+    n = wkv_hip.load_library().rwkv7m_screen_row_groups(rows)
+    return torch.empty(n, 2, C, dtype=torch.float32, device=dev)
+
+
+def norm(x, scale, bias, eps, out_dtype):
+    """LayerNorm over the last axis of x (bf16/fp32) -> (out in out_dtype,
+    mean, rstd fp32 [rows])."""
+    x, scale, bias = _c(x), _f32(scale), _f32(bias)
+    C = x.shape[-1]
+    dev = _check([("x", x, x.shape), ("scale", scale, (C,)),
+                  ("bias", bias, (C,))])
+    rows = x.numel() // C if C else 0
+    out = torch.empty(x.shape, dtype=out_dtype, device=dev)
+    mean = torch.empty(rows, dtype=torch.float32, device=dev)
+    rstd = torch.empty(rows, dtype=torch.float32, device=dev)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_norm", wkv_hip._dtype_code(x),
+          wkv_hip._dtype_code(out), rows, C, P(x), P(scale), P(bias),
+          float(eps), P(out), P(mean), P(rstd), wkv_hip._stream(dev))
+    return out, mean, rstd
+
+
+def norm_backward(x, scale, mean, rstd, dout):
+    """-> (dx like x, d scale, d bias fp32 [C])."""
+    x, scale, dout = _c(x), _f32(scale), _c(dout)
+    C = x.shape[-1]
+    rows = mean.numel()
+    dev = _check([("x", x, x.shape), ("scale", scale, (C,)),
+                  ("mean", mean, (rows,)), ("rstd", rstd, (rows,)),
+                  ("dout", dout, x.shape)])
+    dx, part = torch.empty_like(x), _parts(rows, C, dev)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_norm_backward", wkv_hip._dtype_code(x),
+          wkv_hip._dtype_code(dout), rows, C, P(x), P(scale), P(mean),
+          P(rstd), P(dout), P(dx), P(part), wkv_hip._stream(dev))
+    d = part.sum(0)
+    return dx, d[0], d[1]
+
+
+def unit(x, eps):
+    """x / sqrt(sum x^2 + eps^2) over the last axis, fp32."""
+    x = _c(x)
+    n = x.shape[-1]
+    dev = _check([("x", x, x.shape)])
+    out = torch.empty(x.shape, dtype=torch.float32, device=dev)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_unit", wkv_hip._dtype_code(x),
+          x.numel() // n if n else 0, n, P(x), float(eps), P(out),
+          wkv_hip._stream(dev))
+    return out
+
+
+def unit_backward(x, eps, dout):
+    x, dout = _c(x), _f32(dout)
+    n = x.shape[-1]
+    dev = _check([("x", x, x.shape), ("dout", dout, x.shape)])
+    dx = torch.empty_like(x)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_unit_backward", wkv_hip._dtype_code(x),
+          x.numel() // n if n else 0, n, P(x), float(eps), P(dout), P(dx),
+          wkv_hip._stream(dev))
+    return dx
+
+
+def residual(pre, bias, lam, read, h_base):
+    """h_base + lam sigmoid(pre + bias) read, in h_base's dtype (read's
+    too); lam a device scalar."""
+    pre, read, h_base = _c(pre), _c(read), _c(h_base)
+    bias, lam = _f32(bias), _f32(lam)
+    C = pre.shape[-1]
+    _scalar("lam", lam)
+    dev = _check([("pre", pre, pre.shape), ("bias", bias, (C,)),
+                  ("lam", lam, lam.shape), ("read", read, pre.shape),
+                  ("h_base", h_base, pre.shape)])
+    h = torch.empty_like(h_base)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_residual", wkv_hip._dtype_code(pre),
+          wkv_hip._dtype_code(h), pre.numel() // C if C else 0, C, P(pre),
+          P(bias), P(lam), P(read), P(h_base), P(h), wkv_hip._stream(dev))
+    return h
+
+
+def residual_backward(pre, bias, lam, read, dh):
+    """-> (d_pre like pre, d bias fp32 [C], d lam fp32 scalar, d_read)."""
+    pre, read, dh = _c(pre), _c(read), _c(dh)
+    bias, lam = _f32(bias), _f32(lam)
+    C = pre.shape[-1]
+    _scalar("lam", lam)
+    rows = pre.numel() // C if C else 0
+    dev = _check([("pre", pre, pre.shape), ("bias", bias, (C,)),
+                  ("lam", lam, lam.shape), ("read", read, pre.shape),
+                  ("dh", dh, pre.shape)])
+    d_pre, d_read = torch.empty_like(pre), torch.empty_like(read)
+    part = _parts(rows, C, dev)
+    P = wkv_hip._p
+    _call("rwkv7m_screen_residual_backward", wkv_hip._dtype_code(pre),
+          wkv_hip._dtype_code(dh), rows, C, P(pre), P(bias), P(lam), P(read),
+          P(dh), P(d_pre), P(d_read), P(part), wkv_hip._stream(dev))
+    d = part.sum(0)
+    return d_pre, d[0], d[1].sum(), d_read
+
+
+def stats(rel, rel_w, z_norm, u_norm, upd2, usage0, floor, decay):
+    """-> (usage_T fp32 [B, M], the ten statistics of rwkv7m_screen_stats)."""
+    rel, rel_w, usage0 = _f32(rel), _f32(rel_w), _f32(usage0)
+    z_norm, u_norm, upd2 = _f32(z_norm), _f32(u_norm), _f32(upd2)
+    B, T, M = rel.shape
+    dev = _check([("rel", rel, (B, T, M)), ("rel_w", rel_w, (B, T, M)),
+                  ("z_norm", z_norm, (B, T)), ("u_norm", u_norm, (B, T)),
+                  ("upd2", upd2, (B, T, M, upd2.shape[-1])),
+                  ("usage0", usage0, (B, M))])
+    f = dict(dtype=torch.float32, device=dev)
+    if rel.numel() == 0:  # no steps: the means of nothing
+        out = torch.full((10,), float("nan"), **f)
+        if rel_w is None:
+            out[3:5] = 0.0
+        return usage0.clone(), out
+    part, out, usage = (torch.empty(T, 9, **f), torch.empty(10, **f),
+                        torch.empty(B, M, **f))
+    P = wkv_hip._p
+    _call("rwkv7m_screen_stats", B, T, M, upd2.shape[-1], P(rel), P(rel_w),
+          P(z_norm), P(u_norm), P(upd2), P(usage0), float(floor),
+          float(decay), P(part), P(out), P(usage), wkv_hip._stream(dev))
+    return usage, out

@@ -135,6 +135,7 @@ class _SlotScan(torch.autograd.Function):
         seq, s_t, upd2 = screening_hip.slot_scan(base, slot_term, mu, slots0)
         ctx.save_for_backward(base, slot_term, mu, seq)
         ctx.mark_non_differentiable(upd2)
+        ctx.set_materialize_grads(False)
         return seq, s_t, upd2
 
     @staticmethod
@@ -156,6 +157,7 @@ class _ScreenRead(torch.autograd.Function):
         ctx.save_for_backward(q, proj, tau, age_w)
         ctx.cfg, ctx.dv = cfg, dv
         ctx.mark_non_differentiable(zn, un)
+        ctx.set_materialize_grads(False)
         return u, rel, zn, un
 
     @staticmethod
@@ -209,6 +211,7 @@ class _WriteScan(torch.autograd.Function):
                               mu, s32)
         ctx.floor, ctx.eps = floor, eps
         ctx.mark_non_differentiable(upd2)
+        ctx.set_materialize_grads(False)
         return seq, ages_seq, rel_w, upd2, s_t, a_t
 
     @staticmethod
@@ -233,15 +236,82 @@ class _WriteScan(torch.autograd.Function):
                 d_mu.sum(0).to(mu.dtype), d_s0, d_a0, None, None)
 
 
-def _ema_time_mean(r_bar: torch.Tensor, u0: torch.Tensor,
-                   d: float) -> torch.Tensor:
-    """Mean over t = 0..T-1 of u_t = d u_{t-1} + (1 - d) r_t (u_{-1} = u0),
-    in closed form: (u0 d (1 - d^T) / (1 - d) + sum_t r_t (1 - d^(T-t))) / T
-    (u0 T in place of the first term when d = 1)."""
-    T = r_bar.shape[0]
-    t = torch.arange(T, device=r_bar.device, dtype=r_bar.dtype)
-    head = u0 * (T if d == 1.0 else d * (1.0 - d ** T) / (1.0 - d))
-    return (head + (r_bar * (1.0 - d ** (T - t))).sum()) / T
+class _Norm(torch.autograd.Function):
+    """The screen LayerNorm (fp32 statistics) in the compute dtype."""
+
+    @staticmethod
+    def forward(ctx, x, scale, bias, out_dtype):
+        out, mean, rstd = screening_hip.norm(x, scale, bias, 1e-6, out_dtype)
+        ctx.save_for_backward(x, scale, bias, mean, rstd)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        x, scale, bias, mean, rstd = ctx.saved_tensors
+        dx, ds, db = screening_hip.norm_backward(x, scale, mean, rstd, dout)
+        return dx, ds.to(scale.dtype), db.to(bias.dtype), None
+
+
+class _UnitNorm(torch.autograd.Function):
+    """x / |x| over the last axis, fp32."""
+
+    @staticmethod
+    def forward(ctx, x, eps):
+        ctx.save_for_backward(x)
+        ctx.eps = eps
+        return screening_hip.unit(x, eps)
+
+    @staticmethod
+    def backward(ctx, dout):
+        x, = ctx.saved_tensors
+        return screening_hip.unit_backward(x, ctx.eps, dout), None
+
+
+class _Residual(torch.autograd.Function):
+    """h_base + lam sigmoid(pre + bias) read."""
+
+    @staticmethod
+    def forward(ctx, pre, bias, lam, read, h_base):
+        ctx.save_for_backward(pre, bias, lam, read)
+        return screening_hip.residual(pre, bias, lam, read, h_base)
+
+    @staticmethod
+    def backward(ctx, dh):
+        pre, bias, lam, read = ctx.saved_tensors
+        d_pre, db, dl, d_read = screening_hip.residual_backward(
+            pre, bias, lam, read, dh)
+        return (d_pre, db.to(bias.dtype), dl.reshape(lam.shape).to(lam.dtype),
+                d_read, dh)
+
+
+class _Usage(torch.autograd.Function):
+    """The usage EMA after the last step, and the statistics (not
+    differentiable)."""
+
+    @staticmethod
+    def forward(ctx, rel, rel_w, usage0, zn, un, upd2, floor, decay):
+        usage, stats = screening_hip.stats(rel, rel_w, zn, un, upd2, usage0,
+                                           floor, decay)
+        ctx.save_for_backward(rel, rel_w)
+        ctx.decay = decay
+        ctx.set_materialize_grads(False)
+        ctx.mark_non_differentiable(stats)
+        return usage, stats
+
+    @staticmethod
+    def backward(ctx, du, _d_stats):
+        if du is None:
+            return (None,) * 8
+        rel, rel_w = ctx.saved_tensors
+        d, T = ctx.decay, rel.shape[1]
+        w = (1.0 - d) * d ** torch.arange(T - 1, -1, -1, device=rel.device,
+                                          dtype=torch.float32)
+        d_act = w[None, :, None] * du[:, None]
+        d_w = None
+        if rel_w is not None:  # activity = max(rel, rel_w), ties shared
+            share = (rel > rel_w).float() + 0.5 * (rel == rel_w).float()
+            d_act, d_w = d_act * share, d_act * (1.0 - share)
+        return d_act, d_w, (d ** T) * du, None, None, None, None, None
 
 
 class StateLevelScreening(torch.nn.Module):
@@ -327,15 +397,14 @@ class StateLevelScreening(torch.nn.Module):
         eps = cfg.eps
         B, T, C = x_seq.shape
         cd = self.compute_dtype or x_seq.dtype
-        x_ln = F.layer_norm(x_seq.float(), (C,), self.screen_ln_scale.float(),
-                            self.screen_ln_bias.float(), eps=1e-6).to(cd)
-        q = (x_ln @ self.q_proj_r.to(cd)).float()
-        q = q / torch.sqrt((q * q).sum(-1, keepdim=True) + eps * eps)
+        f32_or_bf16 = (torch.float32, torch.bfloat16)
+        x_in = x_seq if x_seq.dtype in f32_or_bf16 else x_seq.float()
+        x_ln = _Norm.apply(x_in, self.screen_ln_scale, self.screen_ln_bias,
+                           cd)
+        q = _UnitNorm.apply(x_ln @ self.q_proj_r.to(cd), eps)
         tau = 2.0 * torch.sigmoid(self.tau_r_raw.float()) - 1.0
         lam = F.softplus(self.lambda_raw.float())
         mu = self.compute_mu()
-        gate = torch.sigmoid(
-            (x_ln @ self.gate_kernel.to(cd) + self.gate_bias.to(cd)).float())
         dker = self.delta_kernel.to(cd)
         base = (x_ln @ dker[:C] + h_base_seq.to(cd) @ dker[C:2 * C]
                 + self.delta_bias.to(cd))
@@ -344,9 +413,7 @@ class StateLevelScreening(torch.nn.Module):
             # nnx_model.py:1040-1047: the write query and threshold
             q_w = torch.cat([x_ln, h_base_seq.float().to(cd)], -1) @ \
                 self.q_proj_w.to(cd)
-            q_w = q_w.float()
-            q_w = q_w / torch.sqrt((q_w * q_w).sum(-1, keepdim=True)
-                                   + eps * eps)
+            q_w = _UnitNorm.apply(q_w, eps)
             tau_w = 2.0 * torch.sigmoid(self.tau_w_raw.float()) - 1.0
             kw = self.k_proj_w.to(cd)
             seq, ages_seq, rel_w, upd2, slots_t, ages_t = _WriteScan.apply(
@@ -366,39 +433,35 @@ class StateLevelScreening(torch.nn.Module):
         u, rel, zn, un = _ScreenRead.apply(q, proj, tau, age_w, cfg,
                                            cfg.d_v)
         read = (u @ self.out_proj.to(cd)).to(h_base_seq.dtype)
-        h = (h_base_seq.float() + lam * gate * read.float()).to(
-            h_base_seq.dtype)
-        d = float(cfg.usage_ema_decay)
-        activity = rel if rel_w is None else torch.maximum(rel, rel_w)
-        w = (1.0 - d) * d ** torch.arange(T - 1, -1, -1, device=rel.device,
-                                          dtype=torch.float32)
-        usage_t = (d ** T) * state.usage_ema.float() + torch.einsum(
-            "btm,t->bm", activity, w)
+        gate_pre = x_ln @ self.gate_kernel.to(cd)
+        if h_base_seq.dtype in f32_or_bf16:
+            h = _Residual.apply(gate_pre, self.gate_bias, lam, read,
+                                h_base_seq)
+        else:
+            h = _Residual.apply(gate_pre, self.gate_bias, lam, read.float(),
+                                h_base_seq.float()).to(h_base_seq.dtype)
+        usage_t, sv = _Usage.apply(rel, rel_w, state.usage_ema.float(), zn,
+                                   un, upd2, float(cfg.write_rel_floor),
+                                   float(cfg.usage_ema_decay))
         new_state = ScreenState(slots_t.to(state.slots.dtype),
                                 ages_t.to(state.ages.dtype),
                                 usage_t.to(state.usage_ema.dtype))
-        with torch.no_grad():
-            r = rel.detach()
-            zero = torch.zeros((), device=r.device)
-            act = activity.detach()
-            u_mean = _ema_time_mean(act.mean((0, 2)).double(),
-                                    state.usage_ema.double().mean(), d)
-            stats = {
-                "rel_read_mean": r.mean(),
-                "rel_read_max": r.amax(dim=(0, 2)).mean(),
-                "active_slots_mean": (r > 1e-3).sum(-1).float().mean(),
-                "z_norm_mean": zn.mean(),
-                "u_norm_mean": un.mean(),
-                "tau_r": tau.detach(),
-                "lambda_screen": lam.detach(),
-                "rel_write_mean": zero if rel_w is None else rel_w.mean(),
-                "rel_write_effective_mean": (
-                    zero if rel_w is None else torch.clamp(
-                        rel_w, min=cfg.write_rel_floor).mean()),
-                "slot_update_norm_mean": upd2.sum(-1).sqrt().mean(),
-                "slot_usage_ema_mean": u_mean.float(),
-                "tau_w": zero if rel_w is None else tau_w.detach(),
-            }
+        sv = sv.unbind()
+        stats = {
+            "rel_read_mean": sv[0],
+            "rel_read_max": sv[1],
+            "active_slots_mean": sv[2],
+            "z_norm_mean": sv[7],
+            "u_norm_mean": sv[8],
+            "tau_r": tau.detach(),
+            "lambda_screen": lam.detach(),
+            "rel_write_mean": sv[3],
+            "rel_write_effective_mean": sv[4],
+            "slot_update_norm_mean": sv[6],
+            "slot_usage_ema_mean": sv[9],
+            # (without writes the mean write relevance is zero)
+            "tau_w": sv[3] if rel_w is None else tau_w.detach(),
+        }
         return h, new_state, stats
 
 
