@@ -31,7 +31,9 @@ a failed launch raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import os
 import threading
 
@@ -216,6 +218,12 @@ def _dtype_code(t: torch.Tensor) -> int:
 
 
 def _dev(tensors) -> torch.device:
+    # (a decode step is bound by this host code: device indices compare in a
+    # fraction of the time of device objects; -1 is a tensor off the GPU)
+    idx = tensors[0].get_device()
+    if idx >= 0 and all(t.get_device() == idx for t in tensors) and \
+            tensors[0].is_cuda:
+        return tensors[0].device
     dev = tensors[0].device
     for t in tensors:
         if t.device.type != "cuda":
@@ -228,11 +236,28 @@ def _dev(tensors) -> torch.device:
 
 
 def _p(t: torch.Tensor | None):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+# The raw handle of a device's current stream, without building a Stream
+# object where this torch has the call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    if _raw_stream is not None:
+        return _raw_stream(dev.index)
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+_no_switch = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """A context on ``dev``: nothing where it is the current device."""
+    if torch.cuda.current_device() == dev.index:
+        return _no_switch
+    return torch.cuda.device(dev)
 
 
 def _vecs(r, w, k, v, neg_kk, kka):
@@ -242,8 +267,9 @@ def _vecs(r, w, k, v, neg_kk, kka):
                          f" (or [batch, time, ...]), got {tuple(out[0].shape)}")
     # the kernels take bare pointers: every vector must have r's shape and
     # dtype, or they would read past a shorter one
+    shape, dtype = out[0].shape, out[0].dtype
     for x, name in zip(out[1:], ("w", "k", "v", "neg_kk", "kka")):
-        if x.shape != out[0].shape or x.dtype != out[0].dtype:
+        if x.shape != shape or x.dtype != dtype:
             raise ValueError(f"{name} has shape {tuple(x.shape)} and dtype "
                              f"{x.dtype}; expected {tuple(out[0].shape)} "
                              f"{out[0].dtype} like r")
@@ -309,16 +335,20 @@ def set_forward_segments(workgroups_per_head: int) -> None:
     load_library().rwkv7m_debug_set_forward_segments(int(workgroups_per_head))
 
 
+# (these three are functions of their arguments alone)
+@functools.lru_cache(maxsize=256)
 def default_checkpoint_interval(dtype: torch.dtype, head_size: int) -> int:
     code = DTYPE_BF16 if dtype == torch.bfloat16 else DTYPE_F32
     return int(load_library().rwkv7m_wkv7_default_checkpoint_interval(
         code, head_size))
 
 
+@functools.lru_cache(maxsize=1024)
 def checkpoint_count(T: int, interval: int) -> int:
     return int(load_library().rwkv7m_wkv7_checkpoint_count(T, interval))
 
 
+@functools.lru_cache(maxsize=256)
 def checkpoint_dtype(dtype: torch.dtype, head_size: int,
                      interval: int) -> torch.dtype:
     """Element type of the checkpoints for these vectors and interval."""
@@ -344,7 +374,7 @@ def forward(r, w, k, v, neg_kk, kka, initial_state, *, out_state=None,
     s_t = out_state if out_state is not None else torch.empty_like(s0)
     dev = _dev((r, w, k, v, a, b, s0, s_t))
     fn = "rwkv7m_wkv7_forward" + sfx
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = getattr(lib, fn)(
             _dtype_code(r), T, B, H, N, _p(r), _p(w), _p(k), _p(v), _p(a),
             _p(b), _p(s0), _p(y), _p(s_t), _stream(dev))
@@ -367,7 +397,7 @@ def forward_with_aux(r, w, k, v, neg_kk, kka, initial_state, *,
     ckpt = torch.empty((nck, B, H, N, N), device=dev,
                        dtype=checkpoint_dtype(r.dtype, N, ci))
     fn = "rwkv7m_wkv7_forward_with_aux" + sfx
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = getattr(lib, fn)(
             _dtype_code(r), T, B, H, N, _p(r), _p(w), _p(k), _p(v), _p(a),
             _p(b), _p(s0), _p(y), _p(s_t), _p(ckpt), ci, _stream(dev))
@@ -414,7 +444,7 @@ def backward(r, w, k, v, neg_kk, kka, initial_state, dy, ds_t, checkpoints,
             adds.append(None if t is None else t.to(r.dtype).contiguous())
         _dev([r] + [t for t in adds if t is not None])
         fn = "rwkv7m_timemix_wkv_backward"
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = lib.rwkv7m_timemix_wkv_backward(
                 _dtype_code(r), T, B, H, N, _p(r), _p(w), _p(k), _p(v),
                 _p(a), _p(b), _p(s0), _p(dy_c), _p(ds_c), _p(ckpt), ci,
@@ -423,7 +453,7 @@ def backward(r, w, k, v, neg_kk, kka, initial_state, dy, ds_t, checkpoints,
         _check(rc, fn)
         return (*grads, ds0)
     fn = "rwkv7m_wkv7_backward" + sfx
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = getattr(lib, fn)(
             _dtype_code(r), T, B, H, N, _p(r), _p(w), _p(k), _p(v), _p(a),
             _p(b), _p(s0), _p(dy_c), _p(ds_c), _p(ckpt), ci,
@@ -437,23 +467,25 @@ def decode_inplace(r, w, k, v, neg_kk, kka, state):
     [1,B,H,N]. Returns y with the vectors' shape."""
     lib = load_library()
     shape = r.shape
-    r, w, k, v, a, b = _vecs(*(x.reshape(-1, *x.shape[-3:])
-                               for x in (r, w, k, v, neg_kk, kka)))
+    vecs = (r, w, k, v, neg_kk, kka)
+    if r.dim() != 4 or any(x.shape != shape for x in vecs):
+        vecs = [x.reshape(-1, *x.shape[-3:]) for x in vecs]
+    r, w, k, v, a, b = _vecs(*vecs)
     if r.shape[0] != 1 or not state.is_contiguous():
         raise ValueError("decode_inplace takes one token and a contiguous "
                          "state")
     _, B, H, N = r.shape
-    if tuple(state.shape) != (B, H, N, N) or state.dtype != torch.float32:
+    if state.shape != (B, H, N, N) or state.dtype != torch.float32:
         raise ValueError(f"state must be a float32 [{B}, {H}, {N}, {N}] "
                          f"tensor, got {state.dtype} {tuple(state.shape)}")
     dev = _dev((r, w, k, v, a, b, state))
     y = torch.empty_like(r)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.rwkv7m_wkv7_decode_inplace(
             _dtype_code(r), B, H, N, _p(r), _p(w), _p(k), _p(v), _p(a),
             _p(b), _p(state), _p(y), _stream(dev))
     _check(rc, "rwkv7m_wkv7_decode_inplace")
-    return y.reshape(shape)
+    return y if y.shape == shape else y.reshape(shape)
 
 
 def hip_wkv_ffi_backend() -> WKVFFIBackend:

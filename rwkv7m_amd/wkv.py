@@ -23,6 +23,8 @@ Only reverse-mode differentiation is supported (``torch.func.jvp`` raises).
 
 from __future__ import annotations
 
+import inspect
+
 import torch
 
 from .kernels.wkv_backend import resolve_wkv_backend
@@ -188,6 +190,11 @@ class _WKV7(torch.autograd.Function):
             "autodiff (jvp) is not implemented")
 
 
+# apply() binds its arguments to forward's signature on every call; found
+# once, it is read from here.
+_WKV7.forward.__signature__ = inspect.signature(_WKV7.forward)
+
+
 def wkv7(r, w, k, v, neg_kk, kka, initial_state, backend: str | None = None,
          interpret: bool = False):
     """Execute WKV-7 through the selected backend (wkv.py:219-250).
@@ -263,6 +270,10 @@ class _WKV7BatchMajor(torch.autograd.Function):
         raise TypeError(
             "wkv7 supports reverse-mode differentiation only; forward-mode "
             "autodiff (jvp) is not implemented")
+
+
+_WKV7BatchMajor.forward.__signature__ = inspect.signature(
+    _WKV7BatchMajor.forward)
 
 
 def _hip_backend_registered() -> bool:
