@@ -1131,6 +1131,192 @@ int rwkv7m_screen_slot_scan_backward(
                           static_cast<hipStream_t>(stream)));
 }
 
+int rwkv7m_screen_write_deltas(int dtype, int64_t B, int64_t T, int64_t M,
+                               int64_t ds, const void* base,
+                               const float* slot_term, const float* slot_embed,
+                               float* deltas, void* stream) {
+    const char* fn = "rwkv7m_screen_write_deltas";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, 1, 0.0, 0.0));
+    if (B == 0 || T == 0 || M == 0 || ds == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"base", base}, {"slot_term", slot_term},
+                            {"slot_embed", slot_embed}, {"deltas", deltas}}));
+    rwkv7m::ScreenScanWArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.ds = ds;
+    A.base = base;
+    A.slot_term = slot_term;
+    A.slot_embed = slot_embed;
+    A.deltas = deltas;
+    return hip_status("screening write deltas launch",
+                      rwkv7m::launch_screen_write_deltas(
+                          dtype == RWKV7M_DTYPE_BF16, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_write_scan(int dtype, int64_t B, int64_t T, int64_t M,
+                             int64_t ds, int64_t dk, const void* base,
+                             const float* slot_term, const float* slot_embed,
+                             const float* kw, const float* delta_keys,
+                             const float* q_w, const float* tau_w,
+                             const float* mu, double floor, double eps,
+                             const float* slots0, const float* ages0,
+                             void* slots_seq, float* slots32, float* ages_seq,
+                             float* rel_w, float* upd2, float* slots_T,
+                             float* ages_T, float* keys, void* stream) {
+    const char* fn = "rwkv7m_screen_write_scan";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, dk, floor, eps));
+    if (B == 0 || M == 0 || ds == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"slot_term", slot_term},
+                            {"slot_embed", slot_embed}, {"kw", kw},
+                            {"tau_w", tau_w}, {"mu", mu}, {"slots0", slots0},
+                            {"ages0", ages0}, {"slots_T", slots_T},
+                            {"ages_T", ages_T}}));
+    if (T > 0)
+        RWKV7M_TRY(sc_need(fn, {{"base", base}, {"delta_keys", delta_keys},
+                                {"q_w", q_w}, {"slots_seq", slots_seq},
+                                {"slots32", slots32}, {"ages_seq", ages_seq},
+                                {"rel_w", rel_w}, {"upd2", upd2},
+                                {"keys", keys}}));
+    rwkv7m::ScreenScanWArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.ds = ds;
+    A.dk = int(dk);
+    A.floor = float(floor);
+    A.eps = float(eps);
+    A.base = base;
+    A.slot_term = slot_term;
+    A.slot_embed = slot_embed;
+    A.kw = kw;
+    A.delta_keys = delta_keys;
+    A.q_w = q_w;
+    A.tau_w = tau_w;
+    A.mu = mu;
+    A.slots0 = slots0;
+    A.ages0 = ages0;
+    A.slots_seq = slots_seq;
+    A.slots32 = slots32;
+    A.ages_seq = ages_seq;
+    A.rel_w = rel_w;
+    A.upd2 = upd2;
+    A.slots_T = slots_T;
+    A.ages_T = ages_T;
+    A.keys = keys;
+    return hip_status("screening write scan launch",
+                      rwkv7m::launch_screen_write_scan(
+                          dtype == RWKV7M_DTYPE_BF16, false, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_write_keys(int64_t B, int64_t T, int64_t M, int64_t dk,
+                             const float* keys, const float* q_w, double eps,
+                             float* p, float* sim, void* stream) {
+    const char* fn = "rwkv7m_screen_write_keys";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, 1, dk, 0.0, eps));
+    if (B == 0 || T == 0 || M == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"keys", keys}, {"q_w", q_w}, {"p", p},
+                            {"sim", sim}}));
+    rwkv7m::ScreenScanWArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.dk = int(dk);
+    A.eps = float(eps);
+    A.keys = const_cast<float*>(keys);
+    A.q_w = q_w;
+    A.p = p;
+    A.sim = sim;
+    return hip_status("screening write keys launch",
+                      rwkv7m::launch_screen_write_keys(
+                          A, static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_write_scan_backward(
+    int dtype, int64_t B, int64_t T, int64_t M, int64_t ds, const void* base,
+    const float* slot_term, const float* tau_w, const float* mu, double floor,
+    double eps, const float* slots32, const float* sim, const float* wp,
+    const void* d_slots_seq, const float* d_slots_T, const float* d_rel_w,
+    const float* d_ages_seq, const float* d_ages_T, float* d_pre,
+    float* d_slots0, float* d_ages0, float* d_embed_part, float* d_mu_bm,
+    float* d_sim, float* d_tau_w, void* stream) {
+    const char* fn = "rwkv7m_screen_write_scan_backward";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, 1, floor, eps));
+    if (B == 0 || M == 0 || ds == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"slot_term", slot_term}, {"tau_w", tau_w},
+                            {"mu", mu}, {"d_slots0", d_slots0},
+                            {"d_ages0", d_ages0},
+                            {"d_embed_part", d_embed_part},
+                            {"d_mu_bm", d_mu_bm}}));
+    if (T > 0)
+        RWKV7M_TRY(sc_need(fn, {{"base", base}, {"slots32", slots32},
+                                {"sim", sim}, {"wp", wp},
+                                {"d_slots_seq", d_slots_seq},
+                                {"d_pre", d_pre}, {"d_sim", d_sim},
+                                {"d_tau_w", d_tau_w}}));
+    rwkv7m::ScreenScanWArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.ds = ds;
+    A.floor = float(floor);
+    A.eps = float(eps);
+    A.base = base;
+    A.slot_term = slot_term;
+    A.tau_w = tau_w;
+    A.mu = mu;
+    A.slots32 = const_cast<float*>(slots32);
+    A.sim = const_cast<float*>(sim);
+    A.wp = wp;
+    A.d_slots_seq = d_slots_seq;
+    A.d_slots_T = d_slots_T;
+    A.d_rel_w = d_rel_w;
+    A.d_ages_seq = d_ages_seq;
+    A.d_ages_T = d_ages_T;
+    A.d_pre = d_pre;
+    A.d_slots0 = d_slots0;
+    A.d_ages0 = d_ages0;
+    A.d_embed_part = d_embed_part;
+    A.d_mu_bm = d_mu_bm;
+    A.d_sim = d_sim;
+    A.d_tau_w = d_tau_w;
+    return hip_status("screening write scan backward launch",
+                      rwkv7m::launch_screen_write_scan(
+                          dtype == RWKV7M_DTYPE_BF16, true, A,
+                          static_cast<hipStream_t>(stream)));
+}
+
+int rwkv7m_screen_write_queries(int64_t B, int64_t T, int64_t M, int64_t dk,
+                                const float* keys, const float* d_sim,
+                                double eps, float* p, float* dq_w,
+                                void* stream) {
+    const char* fn = "rwkv7m_screen_write_queries";
+    g_last_error.clear();
+    RWKV7M_TRY(sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, 1, dk, 0.0, eps));
+    if (B == 0 || T == 0 || M == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"keys", keys}, {"d_sim", d_sim}, {"p", p},
+                            {"dq_w", dq_w}}));
+    rwkv7m::ScreenScanWArgs A{};
+    A.B = B;
+    A.T = T;
+    A.M = M;
+    A.dk = int(dk);
+    A.eps = float(eps);
+    A.keys = const_cast<float*>(keys);
+    A.d_sim = const_cast<float*>(d_sim);
+    A.p = p;
+    A.dq_w = dq_w;
+    return hip_status("screening write queries launch",
+                      rwkv7m::launch_screen_write_queries(
+                          A, static_cast<hipStream_t>(stream)));
+}
+
 int64_t rwkv7m_screen_row_groups(int64_t rows) {
     g_last_error.clear();
     if (rows < 0) {
