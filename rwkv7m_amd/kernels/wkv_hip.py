@@ -500,13 +500,17 @@ def decode_inplace(r, w, k, v, neg_kk, kka, state):
     return y if y.shape == shape else y.reshape(shape)
 
 
+def _ffi_backward(*args):
+    return backward(*args)
+
+
 def hip_wkv_ffi_backend() -> WKVFFIBackend:
     """The HIP kernels as a reference-contract ``WKVFFIBackend``."""
     load_library()
     return WKVFFIBackend(
         forward=forward,
         forward_with_aux=forward_with_aux,
-        backward=lambda *args: backward(*args),
+        backward=_ffi_backward,
     )
 
 

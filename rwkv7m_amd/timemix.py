@@ -135,6 +135,7 @@ class _TimeMixWKV(torch.autograd.Function):
         ctx.save_for_backward(r_h, w, kp, v_h, nkk, kka, s0, y, w_raw, k, a,
                               g, k_k, k_a, r_k, ln_scale, ln_bias)
         ctx.aux, ctx.N, ctx.eps = tuple(aux), N, eps
+        ctx.set_materialize_grads(False)
         return out, s_t
 
     @staticmethod
@@ -147,7 +148,6 @@ class _TimeMixWKV(torch.autograd.Function):
             raise RuntimeError("time_mix_wkv: backward needs the forward "
                                "run with gradients enabled")
         dout = _zeros_if_none(dout, g)
-        ds_t = _zeros_if_none(ds_t, s0)
         dy, dr_c, dk_c, dv_c, dg, drk, dsc, dbi = timemix_hip.output_backward(
             y, r_h, kp, v_h, g, r_k, ln_scale, ln_bias, dout, N, eps)
         dr, dw, dk_w, dv, dnkk, dkka, ds0 = wkv_hip.backward(

@@ -164,6 +164,7 @@ class _WKV7(torch.autograd.Function):
         *primal, backend, interpret, _ = inputs
         aux = output[2]
         ctx.save_for_backward(*primal)
+        ctx.set_materialize_grads(False)
         ctx.aux = aux
         ctx.backend = backend
         ctx.interpret = interpret
@@ -176,10 +177,15 @@ class _WKV7(torch.autograd.Function):
         r, s0 = inputs[0], inputs[6]
         if dy is None:
             dy = torch.zeros_like(r)
-        if ds_t is None:
+        if ds_t is not None:
+            ds_t = ds_t.to(torch.float32)
+        elif not (resolve_wkv_backend(ctx.backend) == "ffi"
+                  and _hip_backward_registered()):
+            # (the HIP kernels read an absent state cotangent as zeros; other
+            # backends are handed one)
             ds_t = torch.zeros_like(s0)
         grads = _wkv7_backward_dispatch(
-            inputs, (dy.to(r.dtype), ds_t.to(torch.float32)), aux,
+            inputs, (dy.to(r.dtype), ds_t), aux,
             backend=ctx.backend, interpret=ctx.interpret)
         return (*grads, None, None, None)
 
@@ -254,6 +260,7 @@ class _WKV7BatchMajor(torch.autograd.Function):
     @staticmethod
     def setup_context(ctx, inputs, output):
         ctx.save_for_backward(*inputs[:7])
+        ctx.set_materialize_grads(False)
         ctx.aux = output[2]
 
     @staticmethod
@@ -262,6 +269,8 @@ class _WKV7BatchMajor(torch.autograd.Function):
         inputs = ctx.saved_tensors
         aux = ctx.aux
         ctx.aux = None
+        if dy is None:
+            dy = torch.zeros_like(inputs[0])
         grads = wkv_hip.backward(*inputs, dy, ds_t, *aux, layout="bthn")
         return (*grads, None)
 
@@ -280,6 +289,12 @@ def _hip_backend_registered() -> bool:
     from .kernels import wkv_ffi, wkv_hip
     backend = wkv_ffi._registered_backend
     return backend is not None and backend.forward is wkv_hip.forward
+
+
+def _hip_backward_registered() -> bool:
+    from .kernels import wkv_ffi, wkv_hip
+    backend = wkv_ffi._registered_backend
+    return backend is not None and backend.backward is wkv_hip._ffi_backward
 
 
 def wkv7_batch_major(r, w, k, v, neg_kk, kka, initial_state,
