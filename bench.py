@@ -61,10 +61,11 @@ def parse_args():
     p.add_argument("--head-size", type=int, default=0,
                    help="run the configuration at this head size, with H "
                         "scaled to keep H * N (0 = the configuration's N); "
-                        "sizes other than 64 take the sequential kernels")
+                        "16, 32 and 128 take the chunked fp32 kernels, other "
+                        "sizes but 64 the sequential ones")
     p.add_argument("--fp32", action="store_true",
                    help="fp32 vectors instead of the configuration's bf16 "
-                        "(the sequential kernels)")
+                        "(the chunked fp32 kernels)")
     p.add_argument("--layout", choices=("tbhn", "bthn"), default="tbhn",
                    help="vector layout: time-major [T,B,H,N] (the "
                         "reference's WKV contract) or batch-major "
