@@ -821,13 +821,19 @@ f32_bwd_chain_kernel(Args A) {
     for (int c = 0; c < NB; ++c) store4(A.state_out + srow + 16 * c, d[c]);
 }
 
-// The chunk's gradients from S0, D^, X and dU.  A wave owns every fourth
-// block of 16 columns (dr, dw, dk, da, db) and of 16 state rows (dv).
+// The chunk's gradients from S0, D^, X and dU.  A wave owns one block of 16
+// columns (dr, dw, dk, da, db) and of 16 state rows (dv).  Bound by its loads'
+// round trips and the products of the waves that share a SIMD; at N = 128
+// eight waves of 128 registers let two workgroups (73 KB of LDS each) share a
+// CU: 235 -> 115 us a segment (14 chunks of 128 heads, bf16) against four
+// waves with two blocks each and one workgroup a CU.
+template <int N>
+constexpr int kGradWaves = N <= 64 ? 4 : 8;
 template <int N, typename VT>
-__global__ void __launch_bounds__(256, N <= 64 ? 2 : 1)
+__global__ void __launch_bounds__(64 * kGradWaves<N>, N <= 64 ? 2 : 4)
 f32_grads_kernel(Args A) {
     using W = Ws<N, true>;
-    constexpr int NB = W::NB, OWN = (NB + 3) / 4;
+    constexpr int NB = W::NB;
     __shared__ Rows<N> fA, fR, fB, fK, tX, tU, tV, tY;
     __shared__ Mat mat[4];
     __shared__ float zs[N];
@@ -840,33 +846,41 @@ f32_grads_kernel(Args A) {
     const bool valid = t0 + l % 16 < A.T;
     const int64_t toff = (t0 + l % 16) * A.lay.ts + hoff;
 
-    // The state tiles of a wave's column block: in flight from the start
-    // where it has one block (N <= 64), else loaded as they are used.
+    // The state tiles of the wave's column block: in flight from the start,
+    // or (N = 128) once the factors' registers are free, four blocks ahead.
+    // (Buffer loads: the rows' offsets are scalars.)
+    const Rsrc rs = rsrc(s0, N * N * 4), rd = rsrc(ws + W::DH, N * N * 4);
+    const int at0 = (4 * q * N + 16 * (wave < NB ? wave : 0) + l % 16) * 4;
     f4 sc[NB], dc[NB];
-    auto load_state = [&](int c, int b) __attribute__((always_inline)) {
+    auto load_state = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int at = (16 * b + 4 * q + e) * N + 16 * c + l % 16;
-            sc[b][e] = s0[at];
-            dc[b][e] = ws[W::DH + at];
+            const int row = (16 * b + e) * N * 4;
+            sc[b][e] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rs, at0, row, 0));
+            dc[b][e] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rd, at0, row, 0));
         }
     };
-    if constexpr (OWN == 1) {
+    auto load_first = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) load_state(wave < NB ? wave : 0, b);
-    }
-    f4 fP[OWN], fPp[OWN], finv[OWN], few[OWN];
-#pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-        const int c = wave + 4 * o;
-        if (c >= NB) break;
+        for (int b = 0; b < (NB < 4 ? NB : 4); ++b) load_state(b);
+    };
+    if constexpr (NB <= 4) load_first();
+    // (N = 128: a phase's LDS reads stay behind the phase before)
+    auto phase = []() __attribute__((always_inline)) {
+        if constexpr (NB > 4) __builtin_amdgcn_sched_barrier(0);
+    };
+    const int c = wave;
+    f4 fP, fPp, finv, few;
+    if (c < NB) {
         const int col = 16 * c + 4 * q;
         Factors F;
         factors<VT>(F, A, toff + col, valid);
-        fP[o] = F.P;
-        fPp[o] = F.Pp;
-        finv[o] = F.inv;
-        few[o] = F.ew;
+        fP = F.P;
+        fPp = F.Pp;
+        finv = F.inv;
+        few = F.ew;
         fA.put_t(c, l, F.A);
         fR.put_t(c, l, F.R);
         fB.put_t(c, l, F.B);
@@ -882,11 +896,15 @@ f32_grads_kernel(Args A) {
     }
     // (a marked head's values are not used: the loads above stay in bounds)
     if (head_marked(A, bh)) return;
+    phase();
+    if constexpr (NB > 4) load_first();
     __syncthreads();
+    phase();
     // dArb, dArk, dAab, dAak, a wave each
-    mat[wave].put(l, keep_lower(outer<N>(wave < 2 ? tY : tU,
-                                         wave & 1 ? tV : tX, l),
-                                l, wave < 2));
+    if (wave < 4)
+        mat[wave].put(l, keep_lower(outer<N>(wave < 2 ? tY : tU,
+                                             wave & 1 ? tV : tX, l),
+                                    l, wave < 2));
     __syncthreads();
 
     auto put = [&](void* to, const void* add, int64_t off, f4 x) {
@@ -894,22 +912,24 @@ f32_grads_kernel(Args A) {
         if (add) x += load4(static_cast<const VT*>(add) + off);
         store4(static_cast<VT*>(to) + off, x);
     };
-#pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-        const int c = wave + 4 * o;
-        if (c >= NB) break;
+    if (c < NB) {
         // products over the state rows, all T forms: dY S0, dU S0, X D^, V D^
         f4 sr = kZero, sa = kZero, xb = kZero, xk = kZero;
         float z = 0.f;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            if constexpr (OWN > 1) load_state(c, b);
             const f4 s = sc[b], dh = dc[b];
             z += (s[0] * dh[0] + s[1] * dh[1]) + (s[2] * dh[2] + s[3] * dh[3]);
             sr += mm(s, tY.t(b, l));
             sa += mm(s, tU.t(b, l));
             xb += mm(dh, tX.t(b, l));
             xk += mm(dh, tV.t(b, l));
+            if (b + 4 < NB) load_state(b + 4);
+            // (the sums are taken here: left to the end, they held every
+            // block's products in registers)
+            if constexpr (NB > 4)
+                asm volatile("" : "+v"(sr), "+v"(sa), "+v"(xb), "+v"(xk));
+            phase();
         }
         z = add_swap<32>(add_swap<16>(z));  // of column 16c + l % 16
         if (q == 0) zs[16 * c + l % 16] = z;
@@ -922,9 +942,13 @@ f32_grads_kernel(Args A) {
                  ja = fA.jp(c, l);
         const d4 z4 = {0., 0., 0., 0.};
         const d4 pr = mm64(jk, mat[1].dt(l), mm64(jb, mat[0].dt(l), z4));
+        phase();
         const d4 pa = mm64(jk, mat[3].dt(l), mm64(jb, mat[2].dt(l), z4));
+        phase();
         const d4 pb = mm64(ja, mat[2].d(l), mm64(jr, mat[0].d(l), z4));
+        phase();
         const d4 pk = mm64(ja, mat[3].d(l), mm64(jr, mat[1].d(l), z4));
+        phase();
         const f4 tA = fA.t(c, l), tR = fR.t(c, l), tB = fB.t(c, l),
                  tK = fK.t(c, l);
         const f4 p = tB * xb + tK * xk;
@@ -940,22 +964,25 @@ f32_grads_kernel(Args A) {
                 suffix_add(tR[e] * sr[e] +
                            from_right<1>(tA[e] * sa[e], 0.f)) +
                 prefix_add(from_left<1>(p[e], 0.f)) + zt[e];
-            dw[e] = -few[o][e] * dlogd;
-            dR[e] = sr[e] + float(pr[e]);
-            dA[e] = sa[e] + float(pa[e]);
-            dB[e] = xb[e] + float(pb[e]);
-            dK[e] = xk[e] + float(pk[e]);
+            dw[e] = -few[e] * dlogd;
+            // (one rounding where float32 had three)
+            dR[e] = float((sr[e] + pr[e]) * fP[e]);
+            dA[e] = float((sa[e] + pa[e]) * fPp[e]);
+            dB[e] = float((xb[e] + pb[e]) * finv[e]);
+            dK[e] = float((xk[e] + pk[e]) * finv[e]);
         }
         const int64_t off = toff + 16 * c + 4 * q;
-        put(A.dr, A.add_dr, off, dR * fP[o]);
+        put(A.dr, A.add_dr, off, dR);
         put(A.dw, nullptr, off, dw);
-        put(A.dk, A.add_dk, off, dK * finv[o]);
-        put(A.da, nullptr, off, dA * fPp[o]);
-        put(A.db, nullptr, off, dB * finv[o]);
+        put(A.dk, A.add_dk, off, dK);
+        put(A.da, nullptr, off, dA);
+        put(A.db, nullptr, off, dB);
     }
+    phase();
     const f4 ark = load4(ws + W::S + 256 + 4 * l);
     const f4 aak = load4(ws + W::S + 512 + 4 * l);
-    for (int ib = wave; ib < NB; ib += 4) {
+    if (c < NB) {
+        const int ib = c;
         const float* dh = ws + W::DH + (16 * ib + l % 16) * N + 4 * q;
         const f4 x = (mm(tY.j(ib, l), ark) + mm(tU.j(ib, l), aak)) +
                      tree<0, NB>([&](int c) {
@@ -1092,8 +1119,8 @@ hipError_t backward(const SeqBwdArgs& p, hipStream_t stream) {
             (f32_bwd_chain_kernel<N, VT>),
             dim3(unsigned(BH * (N / 16 / kChainWaves<N>))),
             dim3(64 * kChainWaves<N>), 0, stream, A);
-        hipLaunchKernelGGL((f32_grads_kernel<N, VT>), grid, dim3(256), 0,
-                           stream, A);
+        hipLaunchKernelGGL((f32_grads_kernel<N, VT>), grid,
+                           dim3(64 * kGradWaves<N>), 0, stream, A);
         e = hipGetLastError();
         if (e != hipSuccess) break;
         SeqBwdArgs s = p;
