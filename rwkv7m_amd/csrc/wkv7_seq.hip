@@ -605,26 +605,27 @@ wkv7_seq_colsum_kernel(int64_t nt, int64_t t0, int64_t BH, VecLayout lay,
                        VT* dk, VT* da, const int* __restrict__ flags) {
     constexpr int RS = SeqShape<N>::RS;
     const int64_t per = BH * 5 * N;  // values per token
-    const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (e >= nt * per) return;
-    const int64_t tl = e / per;
-    const int64_t rem = e - tl * per;
+    const int64_t rem = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (rem >= per) return;
     const int64_t bh = rem / (5 * N);
     if (flags && !flags[bh]) return;
     const int qj = int(rem - bh * (5 * N));
     const int q = qj / N, j = qj - q * N;
-    float acc = 0.f;
-#pragma unroll
-    for (int sp = 0; sp < RS; ++sp) acc += part[sp * nt * per + e];
-    const int64_t off = (t0 + tl) * lay.ts + lay.head(bh, N) + j;
-    if (q == 1) {
-        const float ew = expf(load_f(w + off));
-        acc *= -ew * expf(-ew);
-    }
-    if (q == 0 && add_dr) acc += load_f(add_dr + off);
-    if (q == 3 && add_dk) acc += load_f(add_dk + off);
     VT* gout[5] = {dr, dw, db, dk, da};
-    store_f(gout[q] + off, acc);
+    for (int64_t tl = blockIdx.y; tl < nt; tl += gridDim.y) {
+        const int64_t e = tl * per + rem;
+        float acc = 0.f;
+#pragma unroll
+        for (int sp = 0; sp < RS; ++sp) acc += part[sp * nt * per + e];
+        const int64_t off = (t0 + tl) * lay.ts + lay.head(bh, N) + j;
+        if (q == 1) {
+            const float ew = expf(load_f(w + off));
+            acc *= -ew * expf(-ew);
+        }
+        if (q == 0 && add_dr) acc += load_f(add_dr + off);
+        if (q == 3 && add_dk) acc += load_f(add_dk + off);
+        store_f(gout[q] + off, acc);
+    }
 }
 
 // Partial column sums held at once by a row-split backward (bytes): the
@@ -714,10 +715,15 @@ hipError_t launch_bwd_nc(const SeqBwdArgs& p, hipStream_t stream) {
                                           c_lo, c_hi, part, t0, t1 - t0,
                                           stream);
             if (e != hipSuccess) break;
-            const int64_t n = (t1 - t0) * BH * 5 * N;
+            // a row of workgroups per token; for marked heads alone, of
+            // which there are hardly ever any, at most 16 rows: a row per
+            // token only to leave at once took 20 us (14 chunks of 128 heads)
+            const int64_t rows = p.flags ? 16 : 65535, nt = t1 - t0;
+            const dim3 grid{unsigned((BH * 5 * N + 255) / 256),
+                            unsigned(nt < rows ? nt : rows)};
             hipLaunchKernelGGL((wkv7_seq_colsum_kernel<N, VT>),
-                               dim3(unsigned((n + 255) / 256)), dim3(256), 0,
-                               stream, t1 - t0, t0, BH, p.lay, part,
+                               grid, dim3(256), 0, stream, nt, t0, BH, p.lay,
+                               part,
                                static_cast<const VT*>(p.w),
                                static_cast<const VT*>(p.add_dr),
                                static_cast<const VT*>(p.add_dk),
