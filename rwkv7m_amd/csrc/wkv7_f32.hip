@@ -33,8 +33,8 @@
 // The sequential kernels spend a token's time on reductions over the columns
 // and rows of the state; here those are the products' sums.  Measured
 // (forward with checkpoints / backward, before -> now): fp32, 96 heads of 64,
-// 512 tokens 183 / 768 -> 111 / 192 us; bf16, 64 heads of 128, 1024 tokens
-// 784 / 3598 -> 417 / 980 us.  Errors against float64 (relative, fp32 vectors,
+// 512 tokens 183 / 768 -> 111 / 188 us; bf16, 64 heads of 128, 1024 tokens
+// 784 / 3598 -> 417 / 655 us.  Errors against float64 (relative, fp32 vectors,
 // the same 96 heads; before): y 1.0e-7 (0.9e-7), S_T 0.8e-7 (0.6e-7), dr
 // 1.0e-7 (1.1e-7), dw 1.2e-7 (1.3e-7), dk 1.0e-7 (1.1e-7), dv 1.1e-7
 // (0.9e-7), da and db 1.5e-7 (1.4e-7).
@@ -823,14 +823,16 @@ f32_bwd_chain_kernel(Args A) {
 
 // The chunk's gradients from S0, D^, X and dU.  A wave owns one block of 16
 // columns (dr, dw, dk, da, db) and of 16 state rows (dv).  Bound by its loads'
-// round trips and the products of the waves that share a SIMD; at N = 128
-// eight waves of 128 registers let two workgroups (73 KB of LDS each) share a
-// CU: 235 -> 115 us a segment (14 chunks of 128 heads, bf16) against four
-// waves with two blocks each and one workgroup a CU.
+// round trips and the products of the waves that share a SIMD, so by the waves
+// in flight: at most 128 registers a lane, for four waves a SIMD.  N = 128,
+// two workgroups of eight waves a CU (73 KB of LDS each): 235 -> 115 us a
+// segment (14 chunks of 128 heads, bf16) against one of four waves with two
+// blocks each; N = 64, four workgroups of four waves a CU (40 KB each): 128 ->
+// 122 us a segment (fp32, B8 T4096 H32) against three.
 template <int N>
 constexpr int kGradWaves = N <= 64 ? 4 : 8;
 template <int N, typename VT>
-__global__ void __launch_bounds__(64 * kGradWaves<N>, N <= 64 ? 2 : 4)
+__global__ void __launch_bounds__(64 * kGradWaves<N>, 4)
 f32_grads_kernel(Args A) {
     using W = Ws<N, true>;
     constexpr int NB = W::NB;
@@ -867,9 +869,9 @@ f32_grads_kernel(Args A) {
         for (int b = 0; b < (NB < 4 ? NB : 4); ++b) load_state(b);
     };
     if constexpr (NB <= 4) load_first();
-    // (N = 128: a phase's LDS reads stay behind the phase before)
+    // (from N = 64 on a phase's LDS reads stay behind the phase before)
     auto phase = []() __attribute__((always_inline)) {
-        if constexpr (NB > 4) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NB >= 4) __builtin_amdgcn_sched_barrier(0);
     };
     const int c = wave;
     f4 fP, fPp, finv, few;
@@ -927,7 +929,7 @@ f32_grads_kernel(Args A) {
             if (b + 4 < NB) load_state(b + 4);
             // (the sums are taken here: left to the end, they held every
             // block's products in registers)
-            if constexpr (NB > 4)
+            if constexpr (NB >= 4)
                 asm volatile("" : "+v"(sr), "+v"(sa), "+v"(xb), "+v"(xk));
             phase();
         }
