@@ -33,11 +33,13 @@
 // The sequential kernels spend a token's time on reductions over the columns
 // and rows of the state; here those are the products' sums.  Measured
 // (forward with checkpoints / backward, before -> now): fp32, 96 heads of 64,
-// 512 tokens 183 / 768 -> 111 / 188 us; bf16, 64 heads of 128, 1024 tokens
-// 784 / 3598 -> 417 / 655 us.  Errors against float64 (relative, fp32 vectors,
-// the same 96 heads; before): y 1.0e-7 (0.9e-7), S_T 0.8e-7 (0.6e-7), dr
-// 1.0e-7 (1.1e-7), dw 1.2e-7 (1.3e-7), dk 1.0e-7 (1.1e-7), dv 1.1e-7
-// (0.9e-7), da and db 1.5e-7 (1.4e-7).
+// 512 tokens 183 / 768 -> 111 / 192 us; bf16, 64 heads of 128, 1024 tokens
+// 784 / 3598 -> 417 / 980 us; more waves in the gradients kernel then took the
+// two training steps from 303 to 299 and from 1416 to 1089 us.  Errors against
+// float64 (relative, fp32 vectors, the same 96 heads; before): y 1.0e-7
+// (0.9e-7), S_T 0.8e-7 (0.6e-7), dr 1.0e-7 (1.1e-7), dw 1.2e-7 (1.3e-7), dk
+// 1.0e-7 (1.1e-7), dv 1.1e-7 (0.9e-7), da and db 1.5e-7 (1.4e-7); with the
+// gradients scaled in float64 the largest of all is 1.4e-7.
 //
 // Range: a chunk with P_L below 2^-60 (no trained decay comes near: the time
 // mix's stays above 2^-14 a chunk), or a non-finite or huge value, is marked
