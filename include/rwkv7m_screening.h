@@ -143,20 +143,6 @@ int rwkv7m_screen_write_backward(
 /* Row groups of the partial sums below for `rows` rows (1 .. 256), or -1. */
 int64_t rwkv7m_screen_row_groups(int64_t rows);
 
-/* out = LayerNorm(x) scale + bias over the C columns of each row; mean, rstd
- * [rows] for the backward. */
-int rwkv7m_screen_norm(int x_dtype, int out_dtype, int64_t rows, int64_t C,
-                       const void *x, const float *scale, const float *bias,
-                       double eps, void *out, float *mean, float *rstd,
-                       void *stream);
-/* dx, and part [row groups][2][C]: summed over the groups, d scale and
- * d bias. */
-int rwkv7m_screen_norm_backward(int x_dtype, int out_dtype, int64_t rows,
-                                int64_t C, const void *x, const float *scale,
-                                const float *mean, const float *rstd,
-                                const void *dout, void *dx, float *part,
-                                void *stream);
-
 /* out = x / sqrt(sum_n x^2 + eps^2) per row, fp32; and its adjoint. */
 int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void *x,
                        double eps, float *out, void *stream);

@@ -1,10 +1,9 @@
 // Elementwise and reduction passes of the screening module around its GEMMs
-// and recurrences (src/rwkv7m/model/nnx_model.py:1015-1160): the screen
-// LayerNorm, unit norms of the queries, the gated residual, and the usage
-// EMA with the statistics.  As single torch operations these were about half
-// of the module's 190 launches per training step, each over a few MB, with a
-// host cost per launch above its device time; every pass here reads its
-// inputs once (the LayerNorm again from cache).  At the 0.185B preset (4096
+// and recurrences (src/rwkv7m/model/nnx_model.py:1015-1160): unit norms of
+// the queries, the gated residual, and the usage EMA with the statistics.  As
+// single torch operations these were about half of the module's 190 launches
+// per training step, each over a few MB, with a host cost per launch above
+// its device time; every pass here reads its inputs once.  At the 0.185B preset (4096
 // rows of 768, bf16) a pass takes 4-11 us (the residual's forward moves its 25
 // MB in 8.2 us, 3.1 TB/s; the final statistics, one block, 19 us), and the
 // read phase's training step goes from 190 launches and 2.37 ms to 109 and
@@ -45,49 +44,6 @@ __device__ __forceinline__ RowLane row_lane() {
             int(threadIdx.x % 64)};
 }
 
-template <typename X, typename O>
-__global__ __launch_bounds__(256) void norm_fwd_kernel(ScreenNormArgs A) {
-    const RowLane p = row_lane();
-    if (p.row >= A.rows) return;
-    const X* x = static_cast<const X*>(A.x) + p.row * A.C;
-    O* o = static_cast<O*>(A.out) + p.row * A.C;
-    float s = 0.f, v = 0.f;
-    for (int64_t c = p.lane; c < A.C; c += 64) s += load_f(x + c);
-    const float mean = wave_total(s) / float(A.C);
-    for (int64_t c = p.lane; c < A.C; c += 64) {
-        const float d = load_f(x + c) - mean;
-        v += d * d;
-    }
-    const float rstd = 1.f / sqrtf(wave_total(v) / float(A.C) + A.eps);
-    for (int64_t c = p.lane; c < A.C; c += 64)
-        store_f(o + c, (load_f(x + c) - mean) * rstd * A.scale[c] + A.bias[c]);
-    if (p.lane == 0) {
-        A.mean[p.row] = mean;
-        A.rstd[p.row] = rstd;
-    }
-}
-
-template <typename X, typename O>
-__global__ __launch_bounds__(256) void norm_bwd_row_kernel(ScreenNormArgs A) {
-    const RowLane p = row_lane();
-    if (p.row >= A.rows) return;
-    const X* x = static_cast<const X*>(A.x) + p.row * A.C;
-    const O* g = static_cast<const O*>(A.dout) + p.row * A.C;
-    X* dx = static_cast<X*>(A.dx) + p.row * A.C;
-    const float mean = A.mean[p.row], rstd = A.rstd[p.row];
-    float s = 0.f, sx = 0.f;
-    for (int64_t c = p.lane; c < A.C; c += 64) {
-        const float d = load_f(g + c) * A.scale[c];
-        s += d;
-        sx += d * ((load_f(x + c) - mean) * rstd);
-    }
-    s = wave_total(s) / float(A.C);
-    sx = wave_total(sx) / float(A.C);
-    for (int64_t c = p.lane; c < A.C; c += 64)
-        store_f(dx + c, rstd * (load_f(g + c) * A.scale[c] - s -
-                                (load_f(x + c) - mean) * rstd * sx));
-}
-
 // 64 columns by the rows blockIdx.y * 4 + wave, + 4 * gridDim.y, ...: `f`
 // gives a row's two values, summed over the rows into part[blockIdx.y][2][C].
 template <typename F>
@@ -108,20 +64,6 @@ __device__ __forceinline__ void column_sums(int64_t rows, int64_t C,
         part[(int64_t(blockIdx.y) * 2 + wave) * C + c] =
             (sum[wave][0][lane] + sum[wave][1][lane]) +
             (sum[wave][2][lane] + sum[wave][3][lane]);
-}
-
-template <typename X, typename O>
-__global__ __launch_bounds__(256) void norm_bwd_param_kernel(
-    ScreenNormArgs A) {
-    const X* x = static_cast<const X*>(A.x);
-    const O* g = static_cast<const O*>(A.dout);
-    column_sums(A.rows, A.C, A.part,
-                [&](int64_t r, int64_t c, float& ds, float& db) {
-                    const float d = load_f(g + r * A.C + c);
-                    ds += d * ((load_f(x + r * A.C + c) - A.mean[r]) *
-                               A.rstd[r]);
-                    db += d;
-                });
 }
 
 template <typename X>
@@ -308,20 +250,6 @@ dim3 col_grid(int64_t C, int64_t groups) {
     return dim3(unsigned((C + 63) / 64), unsigned(groups));
 }
 
-template <typename X, typename O>
-void norm(bool backward, const ScreenNormArgs& A, hipStream_t s) {
-    if (!backward) {
-        hipLaunchKernelGGL((norm_fwd_kernel<X, O>), row_grid(A.rows), dim3(256),
-                           0, s, A);
-        return;
-    }
-    hipLaunchKernelGGL((norm_bwd_row_kernel<X, O>), row_grid(A.rows),
-                       dim3(256), 0, s, A);
-    hipLaunchKernelGGL((norm_bwd_param_kernel<X, O>),
-                       col_grid(A.C, screen_row_groups(A.rows)), dim3(256), 0,
-                       s, A);
-}
-
 template <typename E, typename H>
 void residual(bool backward, const ScreenResidualArgs& A, hipStream_t s) {
     const dim3 grid = col_grid(A.C, screen_row_groups(A.rows));
@@ -341,17 +269,6 @@ void residual(bool backward, const ScreenResidualArgs& A, hipStream_t s) {
 int64_t screen_row_groups(int64_t rows) {
     const int64_t g = (rows + 15) / 16;
     return g < 1 ? 1 : g > 256 ? 256 : g;
-}
-
-hipError_t launch_screen_norm(bool x_bf16, bool out_bf16, bool backward,
-                              const ScreenNormArgs& A, hipStream_t s) {
-    if (x_bf16)
-        out_bf16 ? norm<bf16_t, bf16_t>(backward, A, s)
-                 : norm<bf16_t, float>(backward, A, s);
-    else
-        out_bf16 ? norm<float, bf16_t>(backward, A, s)
-                 : norm<float, float>(backward, A, s);
-    return hipGetLastError();
 }
 
 hipError_t launch_screen_unit(bool bf16, bool backward,

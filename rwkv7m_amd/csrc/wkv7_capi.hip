@@ -1327,65 +1327,6 @@ int64_t rwkv7m_screen_row_groups(int64_t rows) {
     return rwkv7m::screen_row_groups(rows);
 }
 
-int rwkv7m_screen_norm(int x_dtype, int out_dtype, int64_t rows, int64_t C,
-                       const void* x, const float* scale, const float* bias,
-                       double eps, void* out, float* mean, float* rstd,
-                       void* stream) {
-    const char* fn = "rwkv7m_screen_norm";
-    g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, x_dtype, out_dtype, rows, C));
-    if (!(eps >= 0.0))
-        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
-                    std::string(fn) + ": eps must be >= 0");
-    if (rows == 0 || C == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"scale", scale}, {"bias", bias},
-                            {"out", out}, {"mean", mean}, {"rstd", rstd}}));
-    rwkv7m::ScreenNormArgs A{};
-    A.rows = rows;
-    A.C = C;
-    A.eps = float(eps);
-    A.x = x;
-    A.scale = scale;
-    A.bias = bias;
-    A.out = out;
-    A.mean = mean;
-    A.rstd = rstd;
-    return hip_status("screening norm launch",
-                      rwkv7m::launch_screen_norm(
-                          x_dtype == RWKV7M_DTYPE_BF16,
-                          out_dtype == RWKV7M_DTYPE_BF16, false, A,
-                          static_cast<hipStream_t>(stream)));
-}
-
-int rwkv7m_screen_norm_backward(int x_dtype, int out_dtype, int64_t rows,
-                                int64_t C, const void* x, const float* scale,
-                                const float* mean, const float* rstd,
-                                const void* dout, void* dx, float* part,
-                                void* stream) {
-    const char* fn = "rwkv7m_screen_norm_backward";
-    g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, x_dtype, out_dtype, rows, C));
-    if (rows == 0 || C == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"scale", scale}, {"mean", mean},
-                            {"rstd", rstd}, {"dout", dout}, {"dx", dx},
-                            {"part", part}}));
-    rwkv7m::ScreenNormArgs A{};
-    A.rows = rows;
-    A.C = C;
-    A.x = x;
-    A.scale = scale;
-    A.mean = const_cast<float*>(mean);
-    A.rstd = const_cast<float*>(rstd);
-    A.dout = dout;
-    A.dx = dx;
-    A.part = part;
-    return hip_status("screening norm backward launch",
-                      rwkv7m::launch_screen_norm(
-                          x_dtype == RWKV7M_DTYPE_BF16,
-                          out_dtype == RWKV7M_DTYPE_BF16, true, A,
-                          static_cast<hipStream_t>(stream)));
-}
-
 int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void* x,
                        double eps, float* out, void* stream) {
     const char* fn = "rwkv7m_screen_unit";

@@ -235,17 +235,6 @@ hipError_t launch_screen_read(bool bf16, bool backward,
 
 // The screening module's passes around its GEMMs and recurrences
 // (screen_fused.hip).  part: [screen_row_groups(rows)][2][C] partial sums.
-struct ScreenNormArgs {
-    int64_t rows, C;
-    float eps;
-    const void* x;
-    const float *scale, *bias;
-    void* out;
-    float *mean, *rstd;  // [rows]
-    const void* dout;
-    void* dx;
-    float* part;  // d scale, d bias
-};
 struct ScreenUnitArgs {
     int64_t rows, n;
     float eps;
@@ -302,8 +291,6 @@ hipError_t launch_screen_write_keys(const ScreenScanWArgs& A,
 hipError_t launch_screen_write_queries(const ScreenScanWArgs& A,
                                        hipStream_t stream);
 int64_t screen_row_groups(int64_t rows);
-hipError_t launch_screen_norm(bool x_bf16, bool out_bf16, bool backward,
-                              const ScreenNormArgs& A, hipStream_t stream);
 hipError_t launch_screen_unit(bool bf16, bool backward,
                               const ScreenUnitArgs& A, hipStream_t stream);
 hipError_t launch_screen_residual(bool pre_bf16, bool h_bf16, bool backward,

@@ -248,41 +248,6 @@ def _parts(rows, C, dev):
     return torch.empty(n, 2, C, dtype=torch.float32, device=dev)
 
 
-def norm(x, scale, bias, eps, out_dtype):
-    """LayerNorm over the last axis of x (bf16/fp32) -> (out in out_dtype,
-    mean, rstd fp32 [rows])."""
-    x, scale, bias = _c(x), _f32(scale), _f32(bias)
-    C = x.shape[-1]
-    dev = _check([("x", x, x.shape), ("scale", scale, (C,)),
-                  ("bias", bias, (C,))])
-    rows = x.numel() // C if C else 0
-    out = torch.empty(x.shape, dtype=out_dtype, device=dev)
-    mean = torch.empty(rows, dtype=torch.float32, device=dev)
-    rstd = torch.empty(rows, dtype=torch.float32, device=dev)
-    P = wkv_hip._p
-    _call("rwkv7m_screen_norm", wkv_hip._dtype_code(x),
-          wkv_hip._dtype_code(out), rows, C, P(x), P(scale), P(bias),
-          float(eps), P(out), P(mean), P(rstd), wkv_hip._stream(dev))
-    return out, mean, rstd
-
-
-def norm_backward(x, scale, mean, rstd, dout):
-    """-> (dx like x, d scale, d bias fp32 [C])."""
-    x, scale, dout = _c(x), _f32(scale), _c(dout)
-    C = x.shape[-1]
-    rows = mean.numel()
-    dev = _check([("x", x, x.shape), ("scale", scale, (C,)),
-                  ("mean", mean, (rows,)), ("rstd", rstd, (rows,)),
-                  ("dout", dout, x.shape)])
-    dx, part = torch.empty_like(x), _parts(rows, C, dev)
-    P = wkv_hip._p
-    _call("rwkv7m_screen_norm_backward", wkv_hip._dtype_code(x),
-          wkv_hip._dtype_code(dout), rows, C, P(x), P(scale), P(mean),
-          P(rstd), P(dout), P(dx), P(part), wkv_hip._stream(dev))
-    d = part.sum(0)
-    return dx, d[0], d[1]
-
-
 def unit(x, eps):
     """x / sqrt(sum x^2 + eps^2) over the last axis, fp32."""
     x = _c(x)

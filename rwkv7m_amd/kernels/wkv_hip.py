@@ -82,8 +82,6 @@ EXPORTED_SYMBOLS = (
     "rwkv7m_screen_write",
     "rwkv7m_screen_write_backward",
     "rwkv7m_screen_row_groups",
-    "rwkv7m_screen_norm",
-    "rwkv7m_screen_norm_backward",
     "rwkv7m_screen_unit",
     "rwkv7m_screen_unit_backward",
     "rwkv7m_screen_residual",
@@ -193,8 +191,6 @@ def load_library(path: str | None = None):
         lib.rwkv7m_screen_row_groups.restype = i64
         lib.rwkv7m_screen_row_groups.argtypes = [i64]
         for name, args in (
-                ("norm", [i32] * 2 + [i64] * 2 + [vp] * 3 + [f64] + [vp] * 4),
-                ("norm_backward", [i32] * 2 + [i64] * 2 + [vp] * 8),
                 ("unit", [i32] + [i64] * 2 + [vp, f64] + [vp] * 2),
                 ("unit_backward", [i32] + [i64] * 2 + [vp, f64] + [vp] * 3),
                 ("residual", [i32] * 2 + [i64] * 2 + [vp] * 7),

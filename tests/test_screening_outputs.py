@@ -1,0 +1,75 @@
+"""The screening module's outputs where the compute dtype rounds: against the
+same module written with plain torch operations around the recurrence and
+read kernels, in which every intermediate is rounded where torch rounds it.
+A sum taken in another order turns some of the roundings of a bf16
+intermediate, and through the thresholds behind it every gradient moves by
+1e-3; so the states and the output are compared exactly, at the 0.185B preset's
+sizes (of 4096 rows of 768 values some always lie at a rounding's edge).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(dtype, B=8, T=512, C=768, write=False, seed=3):
+    from rwkv7m_amd.screening import (ScreeningConfig, ScreenState,
+                                      StateLevelScreening)
+    cfg = ScreeningConfig(d_model=C, d_slot=128, d_k=64, d_v=64, n_slots=6,
+                          bank_ids=(0, 0, 1, 1, 2, 2),
+                          use_write_screening=write)
+    mod = StateLevelScreening(cfg, compute_dtype=dtype, device="cuda",
+                              seed=seed)
+    g = torch.Generator("cuda").manual_seed(seed)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+
+    with torch.no_grad():
+        mod.gate_bias.copy_(0.5 * normal(C))
+        mod.screen_ln_scale.add_(0.1 * normal(C))
+        mod.screen_ln_bias.add_(0.1 * normal(C))
+    x, h, dh = (normal(B, T, C).to(dtype) for _ in range(3))
+    state = ScreenState(0.3 * normal(B, 6, 128),
+                        torch.zeros(B, 6, device="cuda"),
+                        torch.rand(B, 6, generator=g, device="cuda"))
+    return mod, x.requires_grad_(), h.requires_grad_(), dh, state
+
+
+def _read_phase(mod, x, h, state):
+    """The read-only phase of nnx_model.py:1015-1160 without the usage EMA:
+    (h, slots)."""
+    from rwkv7m_amd import screening as sc
+    cfg, cd, eps, C = mod.config, mod.compute_dtype, mod.config.eps, x.size(-1)
+    x_ln = F.layer_norm(x.float(), (C,), mod.screen_ln_scale.float(),
+                        mod.screen_ln_bias.float(), eps=1e-6).to(cd)
+    q = (x_ln @ mod.q_proj_r.to(cd)).float()
+    q = q / torch.sqrt((q * q).sum(-1, keepdim=True) + eps * eps)
+    gate = torch.sigmoid((x_ln @ mod.gate_kernel.to(cd)
+                          + mod.gate_bias.to(cd)).float())
+    dker = mod.delta_kernel.to(cd)
+    base = (x_ln @ dker[:C] + h.to(cd) @ dker[C:2 * C]
+            + mod.delta_bias.to(cd))
+    term = (mod.slot_embed.to(cd) @ dker[2 * C:]).float()
+    seq, slots, _ = sc._SlotScan.apply(base, term, mod.compute_mu(),
+                                       state.slots.float())
+    kv = torch.cat([mod.k_proj_r, mod.v_proj], dim=1).to(cd)
+    u, _, _, _ = sc._ScreenRead.apply(
+        q, sc._SlotProjection.apply(seq, kv),
+        2.0 * torch.sigmoid(mod.tau_r_raw.float()) - 1.0, None, cfg, cfg.d_v)
+    read = (u @ mod.out_proj.to(cd)).to(h.dtype)
+    lam = F.softplus(mod.lambda_raw.float())
+    return (h.float() + lam * gate * read.float()).to(h.dtype), slots
+
+
+def test_read_phase_slots_round_as_torch(hip_lib):
+    print("case: screening read phase, slots in bf16", flush=True)
+    mod, x, h, _, state = _inputs(torch.bfloat16)
+    _, new, _ = mod(x, h, state)
+    _, slots = _read_phase(mod, x, h, state)
+    torch.cuda.synchronize()
+    assert torch.equal(new.slots, slots)
