@@ -140,28 +140,17 @@ int rwkv7m_screen_write_backward(
  * tensors named after it, everything else fp32.
  */
 
-/* Row groups of the partial sums below for `rows` rows (1 .. 256), or -1. */
-int64_t rwkv7m_screen_row_groups(int64_t rows);
-
-/* out = x / sqrt(sum_n x^2 + eps^2) per row, fp32; and its adjoint. */
-int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void *x,
-                       double eps, float *out, void *stream);
-int rwkv7m_screen_unit_backward(int x_dtype, int64_t rows, int64_t n,
-                                const void *x, double eps, const float *dout,
-                                void *dx, void *stream);
-
-/* h = h_base + lam sigmoid(pre + bias) read; lam one fp32 on the device. */
-int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t rows, int64_t C,
-                           const void *pre, const float *bias,
-                           const float *lam, const void *read,
-                           const void *h_base, void *h, void *stream);
-/* d_pre, d_read, and part [row groups][2][C]: summed over the groups, d bias,
- * and d lam per column. */
-int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t rows,
-                                    int64_t C, const void *pre,
-                                    const float *bias, const float *lam,
+/* h = h_base + lam sigmoid(pre) read over n elements, every operation rounded
+ * to fp32 by itself; lam one fp32 on the device. */
+int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t n,
+                           const void *pre, const float *lam,
+                           const void *read, const void *h_base, void *h,
+                           void *stream);
+/* d_pre, d_read, and d_lam [n], whose sum is lam's gradient. */
+int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t n,
+                                    const void *pre, const float *lam,
                                     const void *read, const void *dh,
-                                    void *d_pre, void *d_read, float *part,
+                                    void *d_pre, void *d_read, float *d_lam,
                                     void *stream);
 
 /*

@@ -1,17 +1,10 @@
 // Elementwise and reduction passes of the screening module around its GEMMs
-// and recurrences (src/rwkv7m/model/nnx_model.py:1015-1160): unit norms of
-// the queries, the gated residual, and the usage EMA with the statistics.  As
-// single torch operations these were about half of the module's 190 launches
-// per training step, each over a few MB, with a host cost per launch above
-// its device time; every pass here reads its inputs once.  At the 0.185B preset (4096
-// rows of 768, bf16) a pass takes 4-11 us (the residual's forward moves its 25
-// MB in 8.2 us, 3.1 TB/s; the final statistics, one block, 19 us), and the
-// read phase's training step goes from 190 launches and 2.37 ms to 109 and
-// 1.87 ms, the write phase's (fp32) from 193 and 2.97 ms to 106 and 2.64 ms.
-//
-// Row passes take a wave per row, lanes over columns; passes that also sum
-// over rows take 64 columns by groups of rows and leave one partial row per
-// group, added by the caller in an order fixed by the shape.
+// and recurrences (src/rwkv7m/model/nnx_model.py:1015-1160): the gated
+// residual, and the usage EMA with the statistics.  As single torch operations
+// these were about fifty launches of a few MB each in a training step, with a
+// host cost per launch above its device time; every pass here reads its inputs
+// once.  At the 0.185B preset (4096 rows of 768) a training step issued op by
+// op goes from 2.35 to 1.89 ms in the read phase (bf16).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,10 +15,6 @@
 namespace rwkv7m {
 namespace {
 
-__device__ __forceinline__ float wave_total(float x) {
-    return add_swap<32>(add_swap<16>(group_sum<16>(x)));
-}
-
 __device__ __forceinline__ float sigmoid(float x) {
     return 1.f / (1.f + expf(-x));
 }
@@ -35,102 +24,40 @@ __device__ __forceinline__ float larger(float a, float b) {
     return a > b || a != a ? a : b;
 }
 
-struct RowLane {
-    int64_t row;
-    int lane;
-};
-__device__ __forceinline__ RowLane row_lane() {
-    return {int64_t(blockIdx.x) * 4 + threadIdx.x / 64,
-            int(threadIdx.x % 64)};
-}
-
-// 64 columns by the rows blockIdx.y * 4 + wave, + 4 * gridDim.y, ...: `f`
-// gives a row's two values, summed over the rows into part[blockIdx.y][2][C].
-template <typename F>
-__device__ __forceinline__ void column_sums(int64_t rows, int64_t C,
-                                            float* part, F f) {
-    __shared__ float sum[2][4][64];
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    const int64_t c = int64_t(blockIdx.x) * 64 + lane;
-    float a = 0.f, b = 0.f;
-    if (c < C)
-        for (int64_t r = int64_t(blockIdx.y) * 4 + wave; r < rows;
-             r += 4 * int64_t(gridDim.y))
-            f(r, c, a, b);
-    sum[0][wave][lane] = a;
-    sum[1][wave][lane] = b;
-    __syncthreads();
-    if (wave < 2 && c < C)
-        part[(int64_t(blockIdx.y) * 2 + wave) * C + c] =
-            (sum[wave][0][lane] + sum[wave][1][lane]) +
-            (sum[wave][2][lane] + sum[wave][3][lane]);
-}
-
-template <typename X>
-__global__ __launch_bounds__(256) void unit_fwd_kernel(ScreenUnitArgs A) {
-    const RowLane p = row_lane();
-    if (p.row >= A.rows) return;
-    const X* x = static_cast<const X*>(A.x) + p.row * A.n;
-    float s = 0.f;
-    for (int64_t c = p.lane; c < A.n; c += 64) s += load_f(x + c) * load_f(x + c);
-    const float norm = sqrtf(wave_total(s) + A.eps * A.eps);
-    for (int64_t c = p.lane; c < A.n; c += 64)
-        A.out[p.row * A.n + c] = load_f(x + c) / norm;
-}
-
-template <typename X>
-__global__ __launch_bounds__(256) void unit_bwd_kernel(ScreenUnitArgs A) {
-    const RowLane p = row_lane();
-    if (p.row >= A.rows) return;
-    const X* x = static_cast<const X*>(A.x) + p.row * A.n;
-    const float* g = A.dout + p.row * A.n;
-    float s = 0.f, d = 0.f;
-    for (int64_t c = p.lane; c < A.n; c += 64) {
-        const float v = load_f(x + c);
-        s += v * v;
-        d += v * g[c];
-    }
-    const float norm = sqrtf(wave_total(s) + A.eps * A.eps);
-    d = wave_total(d) / norm;
-    for (int64_t c = p.lane; c < A.n; c += 64)
-        store_f(static_cast<X*>(A.dx) + p.row * A.n + c,
-                (g[c] - load_f(x + c) / norm * d) / norm);
-}
-
-// h = h_base + lam sigmoid(pre + bias) read
+// h = h_base + lam sigmoid(pre) read, element by element, each operation
+// rounded as torch's separate ones are (no contraction), so that the results
+// and the gradients are theirs bit for bit: in bf16 a coarser or finer sum
+// turns roundings that move some gradients by 1e-3.  The sums over the
+// gradients' elements (of the gate's bias and of lam) are the caller's.
+// Bound by memory: see the file's header for the rate.
 template <typename E, typename H>
 __global__ __launch_bounds__(256) void residual_fwd_kernel(
     ScreenResidualArgs A) {
-    const int64_t c = int64_t(blockIdx.x) * 64 + threadIdx.x % 64;
-    if (c >= A.C) return;
-    const float lam = *A.lam, bias = A.bias[c];
-    for (int64_t r = int64_t(blockIdx.y) * 4 + threadIdx.x / 64; r < A.rows;
-         r += 4 * int64_t(gridDim.y)) {
-        const int64_t i = r * A.C + c;
-        const float g = sigmoid(load_f(static_cast<const E*>(A.pre) + i) + bias);
+#pragma clang fp contract(off)
+    const float lam = *A.lam;
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < A.n;
+         i += 256 * int64_t(gridDim.x)) {
+        const float g = sigmoid(load_f(static_cast<const E*>(A.pre) + i));
+        const float u = lam * g * load_f(static_cast<const H*>(A.read) + i);
         store_f(static_cast<H*>(A.h) + i,
-                load_f(static_cast<const H*>(A.h_base) + i) +
-                    lam * g * load_f(static_cast<const H*>(A.read) + i));
+                load_f(static_cast<const H*>(A.h_base) + i) + u);
     }
 }
 
 template <typename E, typename H>
 __global__ __launch_bounds__(256) void residual_bwd_kernel(
     ScreenResidualArgs A) {
+#pragma clang fp contract(off)
     const float lam = *A.lam;
-    column_sums(A.rows, A.C, A.part,
-                [&](int64_t r, int64_t c, float& db, float& dl) {
-                    const int64_t i = r * A.C + c;
-                    const float g = sigmoid(
-                        load_f(static_cast<const E*>(A.pre) + i) + A.bias[c]);
-                    const float rd = load_f(static_cast<const H*>(A.read) + i);
-                    const float dh = load_f(static_cast<const H*>(A.dh) + i);
-                    const float dp = dh * lam * rd * (g * (1.f - g));
-                    store_f(static_cast<E*>(A.d_pre) + i, dp);
-                    store_f(static_cast<H*>(A.d_read) + i, dh * lam * g);
-                    db += dp;
-                    dl += dh * g * rd;
-                });
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < A.n;
+         i += 256 * int64_t(gridDim.x)) {
+        const float g = sigmoid(load_f(static_cast<const E*>(A.pre) + i));
+        const float dh = load_f(static_cast<const H*>(A.dh) + i);
+        const float dt = dh * load_f(static_cast<const H*>(A.read) + i);
+        store_f(static_cast<H*>(A.d_read) + i, dh * (lam * g));
+        store_f(static_cast<E*>(A.d_pre) + i, dt * lam * (1.f - g) * g);
+        A.d_lam[i] = dt * g;
+    }
 }
 
 // One block per step: sums over (b, m) into part[t][8]: rel, max rel, count
@@ -245,14 +172,11 @@ __global__ __launch_bounds__(256) void stats_final_kernel(ScreenStatsArgs A) {
     }
 }
 
-dim3 row_grid(int64_t rows) { return dim3(unsigned((rows + 3) / 4)); }
-dim3 col_grid(int64_t C, int64_t groups) {
-    return dim3(unsigned((C + 63) / 64), unsigned(groups));
-}
-
 template <typename E, typename H>
 void residual(bool backward, const ScreenResidualArgs& A, hipStream_t s) {
-    const dim3 grid = col_grid(A.C, screen_row_groups(A.rows));
+    // at most 16 workgroups a CU: 3072 elements each at the preset's 3 M
+    const int64_t g = (A.n + 255) / 256;
+    const dim3 grid(unsigned(g < 4096 ? g : 4096));
     if (backward)
         hipLaunchKernelGGL((residual_bwd_kernel<E, H>), grid, dim3(256), 0, s,
                            A);
@@ -262,31 +186,6 @@ void residual(bool backward, const ScreenResidualArgs& A, hipStream_t s) {
 }
 
 }  // namespace
-
-// Row groups of the column sums: 16 rows each, at most 256 groups (with the
-// presets' 12 column tiles 3072 blocks; more groups only lengthen the final
-// addition).
-int64_t screen_row_groups(int64_t rows) {
-    const int64_t g = (rows + 15) / 16;
-    return g < 1 ? 1 : g > 256 ? 256 : g;
-}
-
-hipError_t launch_screen_unit(bool bf16, bool backward,
-                              const ScreenUnitArgs& A, hipStream_t s) {
-    const dim3 grid = row_grid(A.rows);
-    if (backward) {
-        if (bf16)
-            hipLaunchKernelGGL(unit_bwd_kernel<bf16_t>, grid, dim3(256), 0, s, A);
-        else
-            hipLaunchKernelGGL(unit_bwd_kernel<float>, grid, dim3(256), 0, s, A);
-    } else {
-        if (bf16)
-            hipLaunchKernelGGL(unit_fwd_kernel<bf16_t>, grid, dim3(256), 0, s, A);
-        else
-            hipLaunchKernelGGL(unit_fwd_kernel<float>, grid, dim3(256), 0, s, A);
-    }
-    return hipGetLastError();
-}
 
 hipError_t launch_screen_residual(bool pre_bf16, bool h_bf16, bool backward,
                                   const ScreenResidualArgs& A, hipStream_t s) {

@@ -542,21 +542,16 @@ int sc_dims(const char* fn, int dtype, int64_t B, int64_t T, int64_t M,
     return RWKV7M_OK;
 }
 
-// Rows of the fused passes: their grids hold rows / 4 and C / 64 blocks.
-int sc_rows(const char* fn, int dtype_a, int dtype_b, int64_t rows,
-            int64_t C) {
+int sc_elements(const char* fn, int dtype_a, int dtype_b, int64_t n) {
     for (int d : {dtype_a, dtype_b})
         if (d != RWKV7M_DTYPE_F32 && d != RWKV7M_DTYPE_BF16)
             return fail(RWKV7M_ERR_INVALID_ARGUMENT,
                         std::string(fn) + ": tensors must be bfloat16 or "
                                           "float32 (dtype=" +
                             std::to_string(d) + ")");
-    if (rows < 0 || C < 0)
+    if (n < 0)
         return fail(RWKV7M_ERR_INVALID_ARGUMENT,
-                    std::string(fn) + ": negative dimension");
-    if (rows > (int64_t(1) << 25) || C > (int64_t(1) << 25))
-        return fail(RWKV7M_ERR_INVALID_ARGUMENT,
-                    std::string(fn) + ": sizes too large");
+                    std::string(fn) + ": negative size");
     return RWKV7M_OK;
 }
 
@@ -1317,71 +1312,18 @@ int rwkv7m_screen_write_queries(int64_t B, int64_t T, int64_t M, int64_t dk,
                           A, static_cast<hipStream_t>(stream)));
 }
 
-int64_t rwkv7m_screen_row_groups(int64_t rows) {
-    g_last_error.clear();
-    if (rows < 0) {
-        fail(RWKV7M_ERR_INVALID_ARGUMENT,
-             "rwkv7m_screen_row_groups: rows must be >= 0");
-        return -1;
-    }
-    return rwkv7m::screen_row_groups(rows);
-}
-
-int rwkv7m_screen_unit(int x_dtype, int64_t rows, int64_t n, const void* x,
-                       double eps, float* out, void* stream) {
-    const char* fn = "rwkv7m_screen_unit";
-    g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, x_dtype, x_dtype, rows, n));
-    if (rows == 0 || n == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"out", out}}));
-    rwkv7m::ScreenUnitArgs A{};
-    A.rows = rows;
-    A.n = n;
-    A.eps = float(eps);
-    A.x = x;
-    A.out = out;
-    return hip_status("screening unit norm launch",
-                      rwkv7m::launch_screen_unit(
-                          x_dtype == RWKV7M_DTYPE_BF16, false, A,
-                          static_cast<hipStream_t>(stream)));
-}
-
-int rwkv7m_screen_unit_backward(int x_dtype, int64_t rows, int64_t n,
-                                const void* x, double eps, const float* dout,
-                                void* dx, void* stream) {
-    const char* fn = "rwkv7m_screen_unit_backward";
-    g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, x_dtype, x_dtype, rows, n));
-    if (rows == 0 || n == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"x", x}, {"dout", dout}, {"dx", dx}}));
-    rwkv7m::ScreenUnitArgs A{};
-    A.rows = rows;
-    A.n = n;
-    A.eps = float(eps);
-    A.x = x;
-    A.dout = dout;
-    A.dx = dx;
-    return hip_status("screening unit norm backward launch",
-                      rwkv7m::launch_screen_unit(
-                          x_dtype == RWKV7M_DTYPE_BF16, true, A,
-                          static_cast<hipStream_t>(stream)));
-}
-
-int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t rows, int64_t C,
-                           const void* pre, const float* bias,
-                           const float* lam, const void* read,
+int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t n,
+                           const void* pre, const float* lam, const void* read,
                            const void* h_base, void* h, void* stream) {
     const char* fn = "rwkv7m_screen_residual";
     g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, pre_dtype, h_dtype, rows, C));
-    if (rows == 0 || C == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"bias", bias}, {"lam", lam},
-                            {"read", read}, {"h_base", h_base}, {"h", h}}));
+    RWKV7M_TRY(sc_elements(fn, pre_dtype, h_dtype, n));
+    if (n == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"lam", lam}, {"read", read},
+                            {"h_base", h_base}, {"h", h}}));
     rwkv7m::ScreenResidualArgs A{};
-    A.rows = rows;
-    A.C = C;
+    A.n = n;
     A.pre = pre;
-    A.bias = bias;
     A.lam = lam;
     A.read = read;
     A.h_base = h_base;
@@ -1393,30 +1335,27 @@ int rwkv7m_screen_residual(int pre_dtype, int h_dtype, int64_t rows, int64_t C,
                           static_cast<hipStream_t>(stream)));
 }
 
-int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t rows,
-                                    int64_t C, const void* pre,
-                                    const float* bias, const float* lam,
+int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t n,
+                                    const void* pre, const float* lam,
                                     const void* read, const void* dh,
-                                    void* d_pre, void* d_read, float* part,
+                                    void* d_pre, void* d_read, float* d_lam,
                                     void* stream) {
     const char* fn = "rwkv7m_screen_residual_backward";
     g_last_error.clear();
-    RWKV7M_TRY(sc_rows(fn, pre_dtype, h_dtype, rows, C));
-    if (rows == 0 || C == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"bias", bias}, {"lam", lam},
-                            {"read", read}, {"dh", dh}, {"d_pre", d_pre},
-                            {"d_read", d_read}, {"part", part}}));
+    RWKV7M_TRY(sc_elements(fn, pre_dtype, h_dtype, n));
+    if (n == 0) return RWKV7M_OK;
+    RWKV7M_TRY(sc_need(fn, {{"pre", pre}, {"lam", lam}, {"read", read},
+                            {"dh", dh}, {"d_pre", d_pre},
+                            {"d_read", d_read}, {"d_lam", d_lam}}));
     rwkv7m::ScreenResidualArgs A{};
-    A.rows = rows;
-    A.C = C;
+    A.n = n;
     A.pre = pre;
-    A.bias = bias;
     A.lam = lam;
     A.read = read;
     A.dh = dh;
     A.d_pre = d_pre;
     A.d_read = d_read;
-    A.part = part;
+    A.d_lam = d_lam;
     return hip_status("screening residual backward launch",
                       rwkv7m::launch_screen_residual(
                           pre_dtype == RWKV7M_DTYPE_BF16,

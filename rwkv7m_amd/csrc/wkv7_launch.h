@@ -234,24 +234,16 @@ hipError_t launch_screen_read(bool bf16, bool backward,
                               const ScreenReadArgs& A, hipStream_t stream);
 
 // The screening module's passes around its GEMMs and recurrences
-// (screen_fused.hip).  part: [screen_row_groups(rows)][2][C] partial sums.
-struct ScreenUnitArgs {
-    int64_t rows, n;
-    float eps;
-    const void* x;
-    float* out;
-    const float* dout;
-    void* dx;
-};
+// (screen_fused.hip).
 struct ScreenResidualArgs {
-    int64_t rows, C;
+    int64_t n;
     const void* pre;
-    const float *bias, *lam;
+    const float* lam;
     const void *read, *h_base;
     void* h;
     const void* dh;
     void *d_pre, *d_read;
-    float* part;  // d bias, and d lam per column
+    float* d_lam;  // [n]
 };
 struct ScreenStatsArgs {
     int64_t B, T, M, ndw;
@@ -290,9 +282,6 @@ hipError_t launch_screen_write_keys(const ScreenScanWArgs& A,
                                     hipStream_t stream);
 hipError_t launch_screen_write_queries(const ScreenScanWArgs& A,
                                        hipStream_t stream);
-int64_t screen_row_groups(int64_t rows);
-hipError_t launch_screen_unit(bool bf16, bool backward,
-                              const ScreenUnitArgs& A, hipStream_t stream);
 hipError_t launch_screen_residual(bool pre_bf16, bool h_bf16, bool backward,
                                   const ScreenResidualArgs& A,
                                   hipStream_t stream);

@@ -243,72 +243,38 @@ def write_backward(base, slot_term, slot_embed, kw, q_w, tau_w, mu, floor,
     return tuple(outs)
 
 
-def _parts(rows, C, dev):
-    n = wkv_hip.load_library().rwkv7m_screen_row_groups(rows)
-    return torch.empty(n, 2, C, dtype=torch.float32, device=dev)
-
-
-def unit(x, eps):
-    """x / sqrt(sum x^2 + eps^2) over the last axis, fp32."""
-    x = _c(x)
-    n = x.shape[-1]
-    dev = _check([("x", x, x.shape)])
-    out = torch.empty(x.shape, dtype=torch.float32, device=dev)
-    P = wkv_hip._p
-    _call("rwkv7m_screen_unit", wkv_hip._dtype_code(x),
-          x.numel() // n if n else 0, n, P(x), float(eps), P(out),
-          wkv_hip._stream(dev))
-    return out
-
-
-def unit_backward(x, eps, dout):
-    x, dout = _c(x), _f32(dout)
-    n = x.shape[-1]
-    dev = _check([("x", x, x.shape), ("dout", dout, x.shape)])
-    dx = torch.empty_like(x)
-    P = wkv_hip._p
-    _call("rwkv7m_screen_unit_backward", wkv_hip._dtype_code(x),
-          x.numel() // n if n else 0, n, P(x), float(eps), P(dout), P(dx),
-          wkv_hip._stream(dev))
-    return dx
-
-
-def residual(pre, bias, lam, read, h_base):
-    """h_base + lam sigmoid(pre + bias) read, in h_base's dtype (read's
-    too); lam a device scalar."""
-    pre, read, h_base = _c(pre), _c(read), _c(h_base)
-    bias, lam = _f32(bias), _f32(lam)
-    C = pre.shape[-1]
+def residual(pre, lam, read, h_base):
+    """h_base + lam sigmoid(pre) read, in h_base's dtype (read's too); lam a
+    device scalar."""
+    pre, read, h_base, lam = _c(pre), _c(read), _c(h_base), _f32(lam)
     _scalar("lam", lam)
-    dev = _check([("pre", pre, pre.shape), ("bias", bias, (C,)),
-                  ("lam", lam, lam.shape), ("read", read, pre.shape),
-                  ("h_base", h_base, pre.shape)])
+    dev = _check([("pre", pre, pre.shape), ("lam", lam, lam.shape),
+                  ("read", read, pre.shape), ("h_base", h_base, pre.shape)])
+    if read.dtype != h_base.dtype:
+        raise ValueError(f"read is {read.dtype}, h_base {h_base.dtype}")
     h = torch.empty_like(h_base)
     P = wkv_hip._p
     _call("rwkv7m_screen_residual", wkv_hip._dtype_code(pre),
-          wkv_hip._dtype_code(h), pre.numel() // C if C else 0, C, P(pre),
-          P(bias), P(lam), P(read), P(h_base), P(h), wkv_hip._stream(dev))
+          wkv_hip._dtype_code(h), pre.numel(), P(pre), P(lam), P(read),
+          P(h_base), P(h), wkv_hip._stream(dev))
     return h
 
 
-def residual_backward(pre, bias, lam, read, dh):
-    """-> (d_pre like pre, d bias fp32 [C], d lam fp32 scalar, d_read)."""
-    pre, read, dh = _c(pre), _c(read), _c(dh)
-    bias, lam = _f32(bias), _f32(lam)
-    C = pre.shape[-1]
+def residual_backward(pre, lam, read, dh):
+    """-> (d_pre like pre, d_lam fp32 like pre, summed by the caller, d_read
+    like read)."""
+    pre, read, lam = _c(pre), _c(read), _f32(lam)
+    dh = _c(dh).to(read.dtype)
     _scalar("lam", lam)
-    rows = pre.numel() // C if C else 0
-    dev = _check([("pre", pre, pre.shape), ("bias", bias, (C,)),
-                  ("lam", lam, lam.shape), ("read", read, pre.shape),
-                  ("dh", dh, pre.shape)])
+    dev = _check([("pre", pre, pre.shape), ("lam", lam, lam.shape),
+                  ("read", read, pre.shape), ("dh", dh, pre.shape)])
     d_pre, d_read = torch.empty_like(pre), torch.empty_like(read)
-    part = _parts(rows, C, dev)
+    d_lam = torch.empty(pre.shape, dtype=torch.float32, device=dev)
     P = wkv_hip._p
     _call("rwkv7m_screen_residual_backward", wkv_hip._dtype_code(pre),
-          wkv_hip._dtype_code(dh), rows, C, P(pre), P(bias), P(lam), P(read),
-          P(dh), P(d_pre), P(d_read), P(part), wkv_hip._stream(dev))
-    d = part.sum(0)
-    return d_pre, d[0], d[1].sum(), d_read
+          wkv_hip._dtype_code(dh), pre.numel(), P(pre), P(lam), P(read),
+          P(dh), P(d_pre), P(d_read), P(d_lam), wkv_hip._stream(dev))
+    return d_pre, d_lam, d_read
 
 
 def stats(rel, rel_w, z_norm, u_norm, upd2, usage0, floor, decay):

@@ -81,9 +81,6 @@ EXPORTED_SYMBOLS = (
     "rwkv7m_screen_read_backward",
     "rwkv7m_screen_write",
     "rwkv7m_screen_write_backward",
-    "rwkv7m_screen_row_groups",
-    "rwkv7m_screen_unit",
-    "rwkv7m_screen_unit_backward",
     "rwkv7m_screen_residual",
     "rwkv7m_screen_residual_backward",
     "rwkv7m_screen_stats",
@@ -188,13 +185,9 @@ def load_library(path: str | None = None):
         lib.rwkv7m_screen_write.argtypes = wdims + [vp] * 10
         lib.rwkv7m_screen_write_backward.restype = i32
         lib.rwkv7m_screen_write_backward.argtypes = wdims + [vp] * 15
-        lib.rwkv7m_screen_row_groups.restype = i64
-        lib.rwkv7m_screen_row_groups.argtypes = [i64]
         for name, args in (
-                ("unit", [i32] + [i64] * 2 + [vp, f64] + [vp] * 2),
-                ("unit_backward", [i32] + [i64] * 2 + [vp, f64] + [vp] * 3),
-                ("residual", [i32] * 2 + [i64] * 2 + [vp] * 7),
-                ("residual_backward", [i32] * 2 + [i64] * 2 + [vp] * 9),
+                ("residual", [i32] * 2 + [i64] + [vp] * 6),
+                ("residual_backward", [i32] * 2 + [i64] + [vp] * 8),
                 ("write_deltas", [i32] + [i64] * 4 + [vp] * 5),
                 ("write_scan", [i32] + [i64] * 5 + [vp] * 8 + [f64] * 2 +
                  [vp] * 11),

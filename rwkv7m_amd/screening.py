@@ -237,36 +237,21 @@ class _WriteScan(torch.autograd.Function):
                 d_mu.sum(0).to(mu.dtype), d_s0, d_a0, None, None)
 
 
-class _UnitNorm(torch.autograd.Function):
-    """x / |x| over the last axis, fp32."""
-
-    @staticmethod
-    def forward(ctx, x, eps):
-        ctx.save_for_backward(x)
-        ctx.eps = eps
-        return screening_hip.unit(x, eps)
-
-    @staticmethod
-    def backward(ctx, dout):
-        x, = ctx.saved_tensors
-        return screening_hip.unit_backward(x, ctx.eps, dout), None
-
-
 class _Residual(torch.autograd.Function):
-    """h_base + lam sigmoid(pre + bias) read."""
+    """h_base + lam sigmoid(pre) read, rounded as the torch expression in
+    fp32 is."""
 
     @staticmethod
-    def forward(ctx, pre, bias, lam, read, h_base):
-        ctx.save_for_backward(pre, bias, lam, read)
-        return screening_hip.residual(pre, bias, lam, read, h_base)
+    def forward(ctx, pre, lam, read, h_base):
+        ctx.save_for_backward(pre, lam, read)
+        return screening_hip.residual(pre, lam, read, h_base)
 
     @staticmethod
     def backward(ctx, dh):
-        pre, bias, lam, read = ctx.saved_tensors
-        d_pre, db, dl, d_read = screening_hip.residual_backward(
-            pre, bias, lam, read, dh)
-        return (d_pre, db.to(bias.dtype), dl.reshape(lam.shape).to(lam.dtype),
-                d_read, dh)
+        pre, lam, read = ctx.saved_tensors
+        d_pre, d_lam, d_read = screening_hip.residual_backward(pre, lam, read,
+                                                               dh)
+        return d_pre, d_lam.sum_to_size(lam.shape), d_read, dh
 
 
 class _Usage(torch.autograd.Function):
@@ -388,7 +373,10 @@ class StateLevelScreening(torch.nn.Module):
         # pass in its place gained nothing, 1.93 ms a training step either way)
         x_ln = F.layer_norm(x_seq.float(), (C,), self.screen_ln_scale.float(),
                             self.screen_ln_bias.float(), eps=1e-6).to(cd)
-        q = _UnitNorm.apply(x_ln @ self.q_proj_r.to(cd), eps)
+        # (so are the unit norms: a HIP pass turned roundings behind the read,
+        # and gradients moved by 1e-4)
+        q = (x_ln @ self.q_proj_r.to(cd)).float()
+        q = q / torch.sqrt((q * q).sum(-1, keepdim=True) + eps * eps)
         tau = 2.0 * torch.sigmoid(self.tau_r_raw.float()) - 1.0
         lam = F.softplus(self.lambda_raw.float())
         mu = self.compute_mu()
@@ -400,7 +388,9 @@ class StateLevelScreening(torch.nn.Module):
             # nnx_model.py:1040-1047: the write query and threshold
             q_w = torch.cat([x_ln, h_base_seq.float().to(cd)], -1) @ \
                 self.q_proj_w.to(cd)
-            q_w = _UnitNorm.apply(q_w, eps)
+            q_w = q_w.float()
+            q_w = q_w / torch.sqrt((q_w * q_w).sum(-1, keepdim=True)
+                                   + eps * eps)
             tau_w = 2.0 * torch.sigmoid(self.tau_w_raw.float()) - 1.0
             kw = self.k_proj_w.to(cd)
             seq, ages_seq, rel_w, upd2, slots_t, ages_t = _WriteScan.apply(
@@ -420,12 +410,11 @@ class StateLevelScreening(torch.nn.Module):
         u, rel, zn, un = _ScreenRead.apply(q, proj, tau, age_w, cfg,
                                            cfg.d_v)
         read = (u @ self.out_proj.to(cd)).to(h_base_seq.dtype)
-        gate_pre = x_ln @ self.gate_kernel.to(cd)
+        gate_pre = x_ln @ self.gate_kernel.to(cd) + self.gate_bias.to(cd)
         if h_base_seq.dtype in f32_or_bf16:
-            h = _Residual.apply(gate_pre, self.gate_bias, lam, read,
-                                h_base_seq)
+            h = _Residual.apply(gate_pre, lam, read, h_base_seq)
         else:
-            h = _Residual.apply(gate_pre, self.gate_bias, lam, read.float(),
+            h = _Residual.apply(gate_pre, lam, read.float(),
                                 h_base_seq.float()).to(h_base_seq.dtype)
         usage_t, sv = _Usage.apply(rel, rel_w, state.usage_ema.float(), zn,
                                    un, upd2, float(cfg.write_rel_floor),

@@ -3,8 +3,9 @@ same module written with plain torch operations around the recurrence and
 read kernels, in which every intermediate is rounded where torch rounds it.
 A sum taken in another order turns some of the roundings of a bf16
 intermediate, and through the thresholds behind it every gradient moves by
-1e-3; so the states and the output are compared exactly, at the 0.185B preset's
-sizes (of 4096 rows of 768 values some always lie at a rounding's edge).
+1e-3; so the states, the output and every gradient are compared exactly, at the
+0.185B preset's sizes (of 4096 rows of 768 values some always lie at a
+rounding's edge).
 """
 
 from __future__ import annotations
@@ -66,10 +67,17 @@ def _read_phase(mod, x, h, state):
     return (h.float() + lam * gate * read.float()).to(h.dtype), slots
 
 
-def test_read_phase_slots_round_as_torch(hip_lib):
-    print("case: screening read phase, slots in bf16", flush=True)
-    mod, x, h, _, state = _inputs(torch.bfloat16)
-    _, new, _ = mod(x, h, state)
-    _, slots = _read_phase(mod, x, h, state)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_read_phase_equals_torch(hip_lib, dtype):
+    print("case: screening read phase, outputs and gradients", dtype,
+          flush=True)
+    mod, x, h, dh, state = _inputs(dtype)
+    leaves = [x, h, *mod.parameters()]
+    names = ["x", "h_base", *(n for n, _ in mod.named_parameters())]
+    out, new, _ = mod(x, h, state)
+    want, slots = _read_phase(mod, x, h, state)
     torch.cuda.synchronize()
-    assert torch.equal(new.slots, slots)
+    assert torch.equal(out, want) and torch.equal(new.slots, slots)
+    for n, a, b in zip(names, torch.autograd.grad(out, leaves, dh),
+                       torch.autograd.grad(want, leaves, dh)):
+        assert torch.equal(a, b), n
