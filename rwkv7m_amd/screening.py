@@ -249,6 +249,12 @@ class _Residual(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dh):
         pre, lam, read = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph: the same, differentiably
+            g, dhf = torch.sigmoid(pre.float()), dh.float()
+            dt = dhf * read.float()
+            return ((dt * lam * (1.0 - g) * g).to(pre.dtype),
+                    (dt * g).sum_to_size(lam.shape),
+                    (dhf * (lam * g)).to(read.dtype), dh)
         d_pre, d_lam, d_read = screening_hip.residual_backward(pre, lam, read,
                                                                dh)
         return d_pre, d_lam.sum_to_size(lam.shape), d_read, dh

@@ -47,6 +47,31 @@ def test_residual_equals_torch(hip_lib, shape, h_dtype, pre_dtype):
         assert a.dtype == b.dtype and torch.equal(a, b), n
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_residual_second_derivatives(hip_lib, dtype):
+    """Against torch's, to the rounding of sums in another order (fp32: 25
+    terms of 2^-24; bf16 gradients round once more, 2^-8)."""
+    from rwkv7m_amd.screening import _Residual
+    print("case: screening residual, second derivatives", dtype, flush=True)
+    torch.manual_seed(3)
+    leaves = [torch.randn(2, 3, 25).to(dtype).cuda(),
+              torch.tensor(0.3).cuda(), *(torch.randn(2, 3, 25).to(dtype)
+                                          .cuda() for _ in range(2))]
+    pre, lam, read, hb = leaves = [t.requires_grad_() for t in leaves]
+    dh = torch.randn(2, 3, 25).to(dtype).cuda().requires_grad_()
+    out = []
+    for h in (_Residual.apply(*leaves),
+              (hb.float() + lam * torch.sigmoid(pre.float()) * read.float())
+              .to(dtype)):
+        g = torch.autograd.grad(h, leaves[:3], dh, create_graph=True)
+        out.append(torch.autograd.grad([t.float().pow(2).sum() for t in g],
+                                       [*leaves[:3], dh]))
+    tol = 1e-5 if dtype == torch.float32 else 2.0 ** -7
+    for n, a, b in zip(("pre", "lam", "read", "dh"), *out):
+        err = float((a - b).abs().max() / b.abs().max())
+        assert float(b.abs().max()) > 0 and err <= tol, (n, err)
+
+
 @pytest.mark.parametrize("write", [False, True])
 def test_an_empty_call_has_zero_gradients(hip_lib, write):
     from rwkv7m_amd.screening import (ScreeningConfig, StateLevelScreening,
