@@ -282,6 +282,9 @@ def stats(rel, rel_w, z_norm, u_norm, upd2, usage0, floor, decay):
     rel, rel_w, usage0 = _f32(rel), _f32(rel_w), _f32(usage0)
     z_norm, u_norm, upd2 = _f32(z_norm), _f32(u_norm), _f32(upd2)
     B, T, M = rel.shape
+    if B == 0 or M == 0:
+        raise IndexError("the largest relevance of a step needs at least one "
+                         "batch row and slot")
     dev = _check([("rel", rel, (B, T, M)), ("rel_w", rel_w, (B, T, M)),
                   ("z_norm", z_norm, (B, T)), ("u_norm", u_norm, (B, T)),
                   ("upd2", upd2, (B, T, M, upd2.shape[-1])),

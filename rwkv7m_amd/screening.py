@@ -373,7 +373,6 @@ class StateLevelScreening(torch.nn.Module):
         eps = cfg.eps
         B, T, C = x_seq.shape
         cd = self.compute_dtype or x_seq.dtype
-        f32_or_bf16 = (torch.float32, torch.bfloat16)
         # (torch's: in bf16 a LayerNorm with its sums in another order rounds
         # some of x_ln the other way, and every gradient moves by 1e-3; a HIP
         # pass in its place gained nothing, 1.93 ms a training step either way)
@@ -417,14 +416,22 @@ class StateLevelScreening(torch.nn.Module):
                                            cfg.d_v)
         read = (u @ self.out_proj.to(cd)).to(h_base_seq.dtype)
         gate_pre = x_ln @ self.gate_kernel.to(cd) + self.gate_bias.to(cd)
-        if h_base_seq.dtype in f32_or_bf16:
+        if h_base_seq.dtype in (torch.float32, torch.bfloat16) and \
+                h_base_seq.shape == read.shape == gate_pre.shape:
             h = _Residual.apply(gate_pre, lam, read, h_base_seq)
-        else:
-            h = _Residual.apply(gate_pre, lam, read.float(),
-                                h_base_seq.float()).to(h_base_seq.dtype)
-        usage_t, sv = _Usage.apply(rel, rel_w, state.usage_ema.float(), zn,
-                                   un, upd2, float(cfg.write_rel_floor),
-                                   float(cfg.usage_ema_decay))
+        else:  # (h_base_seq broadcasts, or is of another type)
+            h = (h_base_seq.float() + lam * torch.sigmoid(gate_pre.float())
+                 * read.float()).to(h_base_seq.dtype)
+        d, usage0 = float(cfg.usage_ema_decay), state.usage_ema.float()
+        own = usage0
+        if usage0.shape != (B, cfg.n_slots):
+            # it broadcasts: the EMA from its mean, and what is left of the
+            # difference after T steps
+            own = usage0.mean().expand(B, cfg.n_slots)
+        usage_t, sv = _Usage.apply(rel, rel_w, own, zn, un, upd2,
+                                   float(cfg.write_rel_floor), d)
+        if own is not usage0:
+            usage_t = usage_t + (d ** T) * (usage0 - own[0, 0])
         new_state = ScreenState(slots_t.to(state.slots.dtype),
                                 ages_t.to(state.ages.dtype),
                                 usage_t.to(state.usage_ema.dtype))

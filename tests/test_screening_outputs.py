@@ -81,3 +81,51 @@ def test_read_phase_equals_torch(hip_lib, dtype):
     for n, a, b in zip(names, torch.autograd.grad(out, leaves, dh),
                        torch.autograd.grad(want, leaves, dh)):
         assert torch.equal(a, b), n
+
+
+def test_inputs_broadcast_over_the_batch(hip_lib):
+    """h_base_seq, and the usage EMA over the batch and (with one sequence)
+    over more rows, as the torch expressions take them."""
+    print("case: screening, broadcast inputs", flush=True)
+    mod, x, h, _, state = _inputs(torch.float32, B=3, T=20, C=96)
+    one, wide = h.detach()[:1], h.detach()[:1].expand(3, -1, -1).contiguous()
+    outs, grads = [], []
+    for hb in (one, wide):
+        hb = hb.clone().requires_grad_()
+        out, new, _ = mod(x, hb, state)
+        outs.append([out, *new])
+        g, = torch.autograd.grad(out.square().sum(), hb)
+        grads.append(g.sum(0))
+    # (the projection of one batch row's h_base may sum in another order than
+    # three rows': 192 terms of 2^-24)
+    for a, b in zip(*outs):
+        assert torch.allclose(a, b, rtol=1e-5, atol=1e-5)
+    assert torch.allclose(*grads, rtol=1e-5, atol=1e-5)
+
+    def usage(rows, u):
+        u = u.clone().requires_grad_()
+        sub = state._replace(slots=state.slots[:rows], ages=state.ages[:rows],
+                             usage_ema=u)
+        _, new, stats = mod(x[:rows], h[:rows], sub)
+        g, = torch.autograd.grad(new.usage_ema.sum(), u)
+        return new.usage_ema, stats["slot_usage_ema_mean"], g
+
+    u = state.usage_ema
+    got, mean, g = usage(3, u[:1])
+    want, wmean, wg = usage(3, u[:1].expand(3, -1).contiguous())
+    assert got.shape == (3, 6) and torch.allclose(got, want, atol=1e-6)
+    assert torch.allclose(mean, wmean, rtol=1e-5)
+    assert torch.allclose(g, wg.sum(0, keepdim=True), rtol=1e-5)
+    got, mean, g = usage(1, u)
+    assert got.shape == (3, 6)
+    rows = [usage(1, u[i:i + 1]) for i in range(3)]
+    assert torch.allclose(got, torch.cat([r[0] for r in rows]), atol=1e-6)
+    assert torch.allclose(mean, sum(r[1] for r in rows) / 3, rtol=1e-5)
+    assert torch.allclose(g, torch.cat([r[2] for r in rows]), rtol=1e-5)
+
+
+def test_an_empty_batch_is_refused(hip_lib):
+    print("case: screening, no batch rows", flush=True)
+    mod, x, h, _, state = _inputs(torch.float32, B=3, T=4, C=96)
+    with pytest.raises(IndexError):
+        mod(x[:0], h[:0], type(state)(*(t[:0] for t in state)))
