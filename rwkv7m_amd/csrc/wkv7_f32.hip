@@ -557,6 +557,16 @@ __device__ __forceinline__ Rsrc token_rsrc(const VT* base, int64_t ts,
     return rsrc(base, base && n > 0 ? n * ts * int64_t(sizeof(VT)) : 0);
 }
 
+// Tokens from the chunk before chunk ch of a segment, `left` from ch on.  The
+// segment's first chunk has none before it and stays where it is: counted on
+// from there, a segment of one partial chunk would read past the tensor.
+__host__ __device__ constexpr int64_t tokens_from(int64_t left, int64_t ch) {
+    return ch > 0 ? left + 16 : left;
+}
+static_assert(tokens_from(1, 0) == 1 && tokens_from(16, 0) == 16 &&
+                  tokens_from(1, 1) == 17,
+              "a segment of one chunk reads its own tokens only");
+
 __device__ __forceinline__ void fetch(float& x, Rsrc r, int off) {
     x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off * 4, 0, 0));
 }
@@ -772,8 +782,8 @@ f32_bwd_chain_kernel(Args A) {
         lds_barrier();
         feed.load(ws + (ch > 2 ? ch - 2 : 0) * step);
         yp -= A.dy && ch > 0 ? 16 * ts : 0;
-        yb.load(token_rsrc(yp, ts, left + 16), off);
-        left += 16;
+        left = tokens_from(left, ch);
+        yb.load(token_rsrc(yp, ts, left), off);
         __builtin_amdgcn_sched_barrier(0);
         const float* o = ops[buf];
         auto tile = [&](int at) { return load4(o + at + 4 * l); };

@@ -156,3 +156,27 @@ def test_a_value_out_of_range_does_not_reach_earlier_tokens(hip):
     assert torch.isfinite(y[:70]).all() and torch.isfinite(y[:, :, 1]).all()
     rows = torch.arange(64) != 3  # state rows are independent
     assert torch.isfinite(y[:, 0, 0, rows.cuda()]).all()
+
+
+def test_segment_of_one_partial_chunk(hip):
+    """From 915 heads of 128 on the backward's time segments hold one chunk,
+    the last one here one token: the cotangents equal those of the same heads
+    in a call of a few (one segment)."""
+    T, B, H, N, M = 33, 23, 40, 128, 6
+    print("case: chunked fp32 backward, segments of one chunk", flush=True)
+    inp = make_inputs(T, B, H, N, seed=8, state_std=0.1, dstate_std=0.1,
+                      device="cuda", generator="torch")
+    outs = []
+    for bs, hs in ((slice(None), slice(None)), (slice(-1, None),
+                                                slice(-M, None))):
+        x = {n: (t[bs, hs] if n in ("s0", "ds_t") else t[:, bs, hs])
+             .contiguous() for n, t in inp.items()}
+        vecs = [x[n] for n in (*NAMES, "s0")]
+        _, aux = hip.forward_with_aux(*vecs)
+        g = hip.backward(*vecs, x["dy"], x["ds_t"], *aux)
+        assert hip.last_path() == "f32_backward"
+        outs.append([t[-1:, -M:] if n == "ds0" else t[:, -1:, -M:]
+                     for n, t in zip(GRADS, g)])
+    torch.cuda.synchronize()
+    for n, a, b in zip(GRADS, *outs):
+        assert torch.equal(a, b), n
