@@ -1,6 +1,7 @@
 // Chunked WKV-7 in fp32 on the matrix cores (gfx950): fp32 vectors, and bf16
 // vectors with N = 16, 32 or 128, whose arithmetic stays fp32 throughout.
-// Every product is v_mfma_f32_16x16x4_f32; nothing is rounded to 16 bits.
+// The serial products are v_mfma_f32_16x16x4_f32, a chunk's own 16x16 matrices
+// v_mfma_f64_16x16x4_f64; nothing is rounded to 16 bits.
 //
 // A chunk is L = 16 tokens of one head.  With P_t = d_1 ... d_t (per column;
 // P_0 = 1, d = exp(-exp(w))) and
@@ -10,7 +11,7 @@
 // (reference src/rwkv7m/model/rwkv_core.py:54-86) is, over a chunk,
 //     X   = W S0^T + Mak V            W = Minv A~,  Mak = Minv Aak
 //     Y   = R~ S0^T + Arb X + Ark V
-//     S_L = (S0 + X^T B~ + V^T K~) diag(P_L)
+//     S_L = S0 diag(P_L) + X^T B^ + V^T K^    B^_t = b_t P_L / P_t, K^ alike
 // and its reverse (src/rwkv7m/kernels/wkv_pallas_gpu.py:221-257), from the
 // cotangent D of S_L, with D^ = D diag(P_L),
 //     dU  = Wb D^^T + G dY            Wb = Minv^T B~,  G = Minv^T Arb^T
@@ -103,10 +104,13 @@ __device__ __forceinline__ void products(const f4 (&a)[K], const f4 (&b)[K],
     for (int i = 0; i < K; ++i) o[i] = c[i] + d[i];
 }
 
-// The same in float64, whose D tile holds rows 4e + q: with A's rows permuted
-// by i -> 4 (i % 4) + i / 4 (Rows::jp) the result's lanes are as mm's.
+// The same in float64, whose D tile holds rows 4e + q (an H tile): with A's
+// rows permuted by i -> 4 (i % 4) + i / 4 (Rows::jp) the result's lanes are as
+// mm's.  mm64(H tile of M^T, H tile of Y) is an H tile of M Y.
 using d4 = double __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ d4 mm64(f4 a, f4 b, d4 c) {
+constexpr d4 kZero64 = {0., 0., 0., 0.};
+template <typename A, typename B>
+__device__ __forceinline__ d4 mm64(A a, B b, d4 c = kZero64) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], c, 0, 0, 0);
@@ -200,7 +204,7 @@ __device__ __forceinline__ F suffix_add(F x) {
 template <int N, bool BWD>
 struct Ws {
     static constexpr int NB = N / 16;
-    // forward: W, R~ in T form, B~, K~ in J form; Mak, Arb, Ark in T form;
+    // forward: W, R~ in T form, B^, K^ in J form; Mak, Arb, Ark in T form;
     // backward: Wb in T form, A~, R~ in J form; G in T form, Ark, Aak D
     // tiles; then X, dU [16][N] and D^ [N][N]
     static constexpr int M0 = 0, M1 = NB * 256, M2 = 2 * NB * 256,
@@ -238,11 +242,12 @@ __device__ __forceinline__ bool head_marked(const Args& A, int64_t bh) {
 // A lane's 4 columns of the chunk's factors at its token (T form).
 struct Factors {
     f4 A, R, B, K, P, Pp, inv, ew;
+    f4 Bh, Kh;  // B^ = b P_L / P_t, K^ (STATE only)
     bool bad;
 };
 constexpr float kMinP = 0x1p-60f, kMaxFactor = 0x1p90f;
 
-template <typename VT>
+template <typename VT, bool STATE = false>
 __device__ __forceinline__ void factors(Factors& F, const Args& A, int64_t off,
                                         bool valid) {
     f4 r = kZero, w = kZero, k = kZero, a = kZero, b = kZero;
@@ -267,6 +272,11 @@ __device__ __forceinline__ void factors(Factors& F, const Args& A, int64_t off,
         F.R[e] = float(r[e] * p);
         F.B[e] = float(b[e] * inv);
         F.K[e] = float(k[e] * inv);
+        if constexpr (STATE) {
+            const double left = __shfl(p, 15, 16) * inv;
+            F.Bh[e] = float(b[e] * left);
+            F.Kh[e] = float(k[e] * left);
+        }
         // (written so that a NaN fails)
         F.bad |= !(F.P[e] >= kMinP) || !(fabsf(F.A[e]) < kMaxFactor) ||
                  !(fabsf(F.R[e]) < kMaxFactor) ||
@@ -327,15 +337,65 @@ struct Mat {
     }
 };
 
-// sum over columns of x y^T (both in T form): a D tile of the 16x16 product.
+// A 16x16 matrix in float64 between lanes and waves, from an H tile.
+struct Mat64 {
+    double x[16][18];
+    __device__ __forceinline__ void put(int l, d4 h) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * e + l / 16][l % 16] = h[e];
+    }
+    __device__ __forceinline__ d4 h(int l) const {
+        d4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = x[4 * e + l / 16][l % 16];
+        return o;
+    }
+    // an H tile of the transpose
+    __device__ __forceinline__ d4 ht(int l) const {
+        d4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = x[l % 16][4 * e + l / 16];
+        return o;
+    }
+    // rows 4q + e, as mm's tiles: of itself, of the transpose
+    __device__ __forceinline__ d4 d(int l) const {
+        d4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = x[4 * (l / 16) + e][l % 16];
+        return o;
+    }
+    __device__ __forceinline__ d4 dt(int l) const {
+        d4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = x[l % 16][4 * (l / 16) + e];
+        return o;
+    }
+};
+
+// An H tile, rounded, into a D tile's place in the workspace.
+__device__ __forceinline__ void store_tile(float* tile, int l, d4 h) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        tile[4 * (16 * e + l % 16) + l / 16] = float(h[e]);
+}
+
+// sum over columns of x y^T (both in T form): a D tile of the 16x16 product,
+// and an H tile of it in float64.
 template <int N>
 __device__ __forceinline__ f4 outer(const Rows<N>& x, const Rows<N>& y,
                                     int l) {
     return tree<0, N / 16>([&](int c) { return mm(x.t(c, l), y.t(c, l)); });
 }
+template <int N>
+__device__ __forceinline__ d4 outer64(const Rows<N>& x, const Rows<N>& y,
+                                      int l) {
+    d4 o = kZero64;
+#pragma unroll
+    for (int c = 0; c < N / 16; ++c) o = mm64(x.t(c, l), y.t(c, l), o);
+    return o;
+}
 
-// D tile entries with row (`rows`: 4q + e) > column, or >= with the diagonal,
-// of a matrix or (upper) of its transpose.
+// D tile entries with row (4q + e) > column, or >= with the diagonal.
 __device__ __forceinline__ f4 keep_lower(f4 d, int l, bool diag) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -344,28 +404,38 @@ __device__ __forceinline__ f4 keep_lower(f4 d, int l, bool diag) {
     }
     return d;
 }
-__device__ __forceinline__ f4 keep_upper(f4 d, int l, bool diag) {
+// The same of an H tile (rows 4e + q), and of a matrix's transpose (upper).
+__device__ __forceinline__ d4 keep_lower(d4 h, int l, bool diag) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int i = 4 * (l / 16) + e, j = l % 16;
-        d[e] = (i < j || (diag && i == j)) ? d[e] : 0.f;
+        const int i = 4 * e + l / 16, j = l % 16;
+        h[e] = (i > j || (diag && i == j)) ? h[e] : 0.;
     }
-    return d;
+    return h;
+}
+__device__ __forceinline__ d4 keep_upper(d4 h, int l, bool diag) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int i = 4 * e + l / 16, j = l % 16;
+        h[e] = (i < j || (diag && i == j)) ? h[e] : 0.;
+    }
+    return h;
 }
 
-// (I - A)^-1 of a strictly lower 16x16 A and its transpose:
-// (I + A)(I + A^2)(I + A^4)(I + A^8), A nilpotent.  at: D tile of A^T.
-__device__ __forceinline__ void inverse(f4 a, f4 at, int l, f4& m, f4& mt) {
-    f4 one;
+// (I - A)^-1 of a strictly lower 16x16 A:
+// (I + A)(I + A^2)(I + A^4)(I + A^8), A nilpotent.  a, at: H tiles of A and
+// A^T.  In float64: with keys that resemble each other A is near -1 below the
+// diagonal, the powers reach 3e3 and cancel to O(1), which in float32 left y
+// and the gradients 1e-5 to 1e-4 off.
+__device__ __forceinline__ d4 inverse(d4 a, d4 at, int l) {
+    d4 one;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) one[e] = 4 * (l / 16) + e == l % 16 ? 1.f : 0.f;
-    const f4 a2 = mm(at, a), a2t = mm(a, at);
-    const f4 q1 = one + a + mm(at, a2, a2), q1t = one + at + mm(a2, at, a2t);
-    const f4 a4 = mm(a2t, a2), a4t = mm(a2, a2t);
-    const f4 q2 = mm(q1t, a4, q1), q2t = mm(a4, q1t, q1t);
-    const f4 a8 = mm(a4t, a4);
-    m = mm(q2t, a8, q2);
-    mt = mm(a8, q2t, q2t);
+    for (int e = 0; e < 4; ++e) one[e] = 4 * e + l / 16 == l % 16 ? 1. : 0.;
+    const d4 a2 = mm64(at, a), a2t = mm64(a, at);
+    const d4 q1 = one + a + mm64(at, a2, a2), q1t = one + at + mm64(a2, at, a2t);
+    const d4 a4 = mm64(a2t, a2), a4t = mm64(a2, a2t);
+    const d4 q2 = mm64(q1t, a4, q1), q2t = mm64(a4, q1t, q1t);
+    return mm64(q2t, mm64(a4t, a4), q2);
 }
 
 // One workgroup per chunk and head: bound by the inverse's six dependent
@@ -376,7 +446,9 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     using W = Ws<N, BWD>;
     constexpr int NB = W::NB;
     __shared__ Rows<N> fA, fR, fB, fK;
-    __shared__ Mat mat[3];
+    __shared__ Rows<BWD ? 16 : N> fBh, fKh;
+    __shared__ Mat64 sA, sM;
+    __shared__ Mat sMak;
     __shared__ f4 sW[BWD ? NB : 1][64];
     const int64_t bh = blockIdx.x, ch = blockIdx.y;
     const int wave = threadIdx.x / 64, l = threadIdx.x % 64;
@@ -391,7 +463,7 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     for (int c = wave; c < NB; c += 4) {
         const int col = 16 * c + 4 * q;
         Factors F;
-        factors<VT>(F, A, toff + col, valid);
+        factors<VT, !BWD>(F, A, toff + col, valid);
         bad |= F.bad;
         if (valid) {
             bad |= out_of_range(
@@ -404,6 +476,10 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
         fR.put_t(c, l, F.R);
         fB.put_t(c, l, F.B);
         fK.put_t(c, l, F.K);
+        if constexpr (!BWD) {
+            fBh.put_t(c, l, F.Bh);
+            fKh.put_t(c, l, F.Kh);
+        }
         if (l % 16 == 15) store4(ws + W::PL + col, F.P);
     }
     // (a barrier: the factors are complete)
@@ -411,67 +487,69 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     if (threadIdx.x == 0) A.flags[ch * A.BH + bh] = bad;
     if (bad) return;
 
-    // The four matrices, a wave each; D tiles of Aab, Aak, Arb^T, and Ark^T
-    // (forward) or Ark (backward).
-    f4 m;
+    // The four matrices, a wave each; H tiles of Aab, Aak, Arb^T, and Ark^T
+    // (forward) or Ark (backward).  In float64 from the rounded factors, and
+    // rounded once where they are stored: in float32 their sums' error,
+    // times what the inverse and the serial step make of it, was most of y's.
+    d4 m;
     if (wave == 0)
-        m = keep_lower(outer<N>(fA, fB, l), l, false);
+        m = keep_lower(outer64<N>(fA, fB, l), l, false);
     else if (wave == 1)
-        m = keep_lower(outer<N>(fA, fK, l), l, false);
+        m = keep_lower(outer64<N>(fA, fK, l), l, false);
     else if (wave == 2)
-        m = keep_upper(outer<N>(fB, fR, l), l, true);
+        m = keep_upper(outer64<N>(fB, fR, l), l, true);
     else if (!BWD)
-        m = keep_upper(outer<N>(fK, fR, l), l, true);
+        m = keep_upper(outer64<N>(fK, fR, l), l, true);
     else
-        m = keep_lower(outer<N>(fR, fK, l), l, true);
+        m = keep_lower(outer64<N>(fR, fK, l), l, true);
     if (wave == 0) {
-        f4 minv, minvt;
-        mat[2].put(l, m);
+        sA.put(l, m);
         __builtin_amdgcn_wave_barrier();
-        inverse(m, mat[2].dt(l), l, minv, minvt);
-        mat[0].put(l, minv);
-        mat[1].put(l, minvt);
+        sM.put(l, inverse(m, sA.ht(l), l));
     } else {
         // meanwhile the operands that need no inverse
         for (int c = wave - 1; c < NB; c += 3) {
             if (!BWD) {
                 store4(ws + W::M1 + c * 256 + 4 * l, fR.t(c, l));
-                store4(ws + W::M2 + c * 256 + 4 * l, fB.j(c, l));
-                store4(ws + W::M3 + c * 256 + 4 * l, fK.j(c, l));
+                store4(ws + W::M2 + c * 256 + 4 * l, fBh.j(c, l));
+                store4(ws + W::M3 + c * 256 + 4 * l, fKh.j(c, l));
             } else {
                 store4(ws + W::M1 + c * 256 + 4 * l, fA.j(c, l));
                 store4(ws + W::M2 + c * 256 + 4 * l, fR.j(c, l));
             }
         }
-        if (!BWD && wave >= 2)
-            store4(ws + W::S + (wave - 1) * 256 + 4 * l, m);
-        if (BWD && wave == 3) store4(ws + W::S + 256 + 4 * l, m);
-        if (BWD && wave == 1) store4(ws + W::S + 512 + 4 * l, m);
+        if (!BWD && wave >= 2) store_tile(ws + W::S + (wave - 1) * 256, l, m);
+        if (BWD && wave == 3) store_tile(ws + W::S + 256, l, m);
+        if (BWD && wave == 1) store_tile(ws + W::S + 512, l, m);
     }
     __syncthreads();
-    const f4 minv = mat[0].d(l), minvt = mat[1].d(l);
     for (int c = wave; c < NB; c += 4) {
-        const f4 wt = mm(fA.j(c, l), minvt);
+        const f4 wt =
+            __builtin_convertvector(mm64(fA.jp(c, l), sM.dt(l)), f4);
         if (!BWD) {
             store4(ws + W::M0 + c * 256 + 4 * l, wt);
         } else {
             sW[c][l] = wt;
-            store4(ws + W::M0 + c * 256 + 4 * l, mm(fB.j(c, l), minv));
+            store4(ws + W::M0 + c * 256 + 4 * l,
+                   __builtin_convertvector(mm64(fB.jp(c, l), sM.d(l)), f4));
         }
     }
     if (wave == 1) {
-        const f4 mak = mm(m, minvt);  // T form of Minv Aak
-        if (!BWD)
-            store4(ws + W::S + 4 * l, mak);
-        else
-            mat[2].put(l, mak);
+        const d4 mak = mm64(m, sM.ht(l));  // T form of Minv Aak
+        if (!BWD) {
+            store_tile(ws + W::S, l, mak);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sMak.x[4 * e + q][l % 16] = float(mak[e]);
+        }
     }
     if (BWD && wave == 2)
-        store4(ws + W::S + 4 * l, mm(m, minv));  // T form of G
+        store_tile(ws + W::S, l, mm64(m, sM.h(l)));  // T form of G
     if constexpr (BWD) {
         // X = W S0^T + Mak V, 16 state rows a wave
         __syncthreads();
-        const f4 mak = mat[2].d(l);
+        const f4 mak = sMak.d(l);
         for (int ib = wave; ib < NB; ib += 4) {
             const int row = 16 * ib + l % 16;
             const float* s0 =
@@ -716,8 +794,9 @@ f32_fwd_chain_kernel(Args A) {
             products(bk, xv, up);
 #pragma unroll
             for (int c = 0; c < G; ++c)
-                s[c0 + c] = (s[c0 + c] + (up[2 * c] + up[2 * c + 1])) *
-                            load4(o + W::PL + 16 * (c0 + c) + 4 * q);
+                s[c0 + c] = s[c0 + c] *
+                                load4(o + W::PL + 16 * (c0 + c) + 4 * q) +
+                            (up[2 * c] + up[2 * c + 1]);
         }
         y += yx;
         // (the loads' values are taken before the stores are issued: memory
@@ -954,14 +1033,13 @@ f32_grads_kernel(Args A) {
         // far from float64 as the rest).
         const f4 jb = fB.jp(c, l), jk = fK.jp(c, l), jr = fR.jp(c, l),
                  ja = fA.jp(c, l);
-        const d4 z4 = {0., 0., 0., 0.};
-        const d4 pr = mm64(jk, mat[1].dt(l), mm64(jb, mat[0].dt(l), z4));
+        const d4 pr = mm64(jk, mat[1].dt(l), mm64(jb, mat[0].dt(l)));
         phase();
-        const d4 pa = mm64(jk, mat[3].dt(l), mm64(jb, mat[2].dt(l), z4));
+        const d4 pa = mm64(jk, mat[3].dt(l), mm64(jb, mat[2].dt(l)));
         phase();
-        const d4 pb = mm64(ja, mat[2].d(l), mm64(jr, mat[0].d(l), z4));
+        const d4 pb = mm64(ja, mat[2].d(l), mm64(jr, mat[0].d(l)));
         phase();
-        const d4 pk = mm64(ja, mat[3].d(l), mm64(jr, mat[1].d(l), z4));
+        const d4 pk = mm64(ja, mat[3].d(l), mm64(jr, mat[1].d(l)));
         phase();
         const f4 tA = fA.t(c, l), tR = fR.t(c, l), tB = fB.t(c, l),
                  tK = fK.t(c, l);
