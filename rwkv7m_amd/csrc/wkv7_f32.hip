@@ -1,7 +1,8 @@
 // Chunked WKV-7 in fp32 on the matrix cores (gfx950): fp32 vectors, and bf16
 // vectors with N = 16, 32 or 128, whose arithmetic stays fp32 throughout.
-// The serial products are v_mfma_f32_16x16x4_f32, a chunk's own 16x16 matrices
-// v_mfma_f64_16x16x4_f64; nothing is rounded to 16 bits.
+// The products are v_mfma_f32_16x16x4_f32, those of a chunk's own 16x16 matrices
+// and of the state's and its cotangent's update v_mfma_f64_16x16x4_f64; nothing
+// is rounded to 16 bits.
 //
 // A chunk is L = 16 tokens of one head.  With P_t = d_1 ... d_t (per column;
 // P_0 = 1, d = exp(-exp(w))) and
@@ -34,13 +35,19 @@
 // The sequential kernels spend a token's time on reductions over the columns
 // and rows of the state; here those are the products' sums.  Measured
 // (forward with checkpoints / backward, before -> now): fp32, 96 heads of 64,
-// 512 tokens 183 / 768 -> 111 / 192 us; bf16, 64 heads of 128, 1024 tokens
-// 784 / 3598 -> 417 / 980 us; more waves in the gradients kernel then took the
-// two training steps from 303 to 299 and from 1416 to 1089 us.  Errors against
-// float64 (relative, fp32 vectors, the same 96 heads; before): y 1.0e-7
-// (0.9e-7), S_T 0.8e-7 (0.6e-7), dr 1.0e-7 (1.1e-7), dw 1.2e-7 (1.3e-7), dk
-// 1.0e-7 (1.1e-7), dv 1.1e-7 (0.9e-7), da and db 1.5e-7 (1.4e-7); with the
-// gradients scaled in float64 the largest of all is 1.4e-7.
+// 512 tokens 183 / 768 -> 140 / 200 us; bf16, 64 heads of 128, 1024 tokens
+// 784 / 3598 -> 480 / 750 us.  Of that the float64 products are 44 and 139 us;
+// without them (all float32) the errors below grew to what is said at
+// `inverse` and at the chains.
+//
+// Errors against float64 (2-norm, fp32 vectors, 4 heads of 64, 512 tokens; in
+// 1e-7, the sequential kernels' in brackets): independent keys as a model's
+// y 0.8 (0.9), S_T 0.4 (0.6), dr 0.9 (1.0), dw 1.2 (1.3), dk 0.9 (1.1), dv 0.9
+// (0.9), da 1.2 (1.4), db 1.2 (1.4), dS0 0.5 (0.6); keys within 0.1 of one
+// direction, a near 0.95, slow decay y 2.0 (1.2), S_T 1.6 (1.1), dr 2.3 (1.4),
+// dw 2.6 (1.8), dk 1.0 (1.3), dv 2.4 (2.0), da 2.6 (2.4), db 1.2 (1.4), dS0
+// 0.6 (1.0); one key repeated, hardly any decay y 5.4 (4.6), S_T 6.2 (5.9),
+// the gradients 5.6 to 11 (4.7 to 12).  The other head sizes are alike.
 //
 // Range: a chunk with P_L below 2^-60 (no trained decay comes near: the time
 // mix's stays above 2^-14 a chunk), or a non-finite or huge value, is marked
@@ -438,15 +445,15 @@ __device__ __forceinline__ d4 inverse(d4 a, d4 at, int l) {
     return mm64(q2t, mm64(a4t, a4), q2);
 }
 
-// One workgroup per chunk and head: bound by the inverse's six dependent
-// products on one wave (about 3,000 cycles), hidden by the other chunks'
-// workgroups on the CU (18 KB of LDS each at N = 64).
+// One workgroup per chunk and head: bound by the inverse's products on one
+// wave, ten in float64 of which four follow each other, hidden by the other
+// chunks' workgroups on the CU (24 KB of LDS each at N = 64).  96 heads of 64,
+// 32 chunks: forward 40, backward 50 us (all float32: 31 and 43).
 template <int N, typename VT, bool BWD>
 __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     using W = Ws<N, BWD>;
     constexpr int NB = W::NB;
     __shared__ Rows<N> fA, fR, fB, fK;
-    __shared__ Rows<BWD ? 16 : N> fBh, fKh;
     __shared__ Mat64 sA, sM;
     __shared__ Mat sMak;
     __shared__ f4 sW[BWD ? NB : 1][64];
@@ -459,9 +466,13 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     const bool valid = t0 + l % 16 < A.T;
     const int64_t toff = (t0 + l % 16) * A.lay.ts + hoff;
 
+    constexpr int PER = (NB + 3) / 4;  // column blocks of a wave
+    f4 Bh[PER], Kh[PER];
     bool bad = false;
-    for (int c = wave; c < NB; c += 4) {
-        const int col = 16 * c + 4 * q;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int c = wave + 4 * i, col = 16 * c + 4 * q;
+        if (c >= NB) break;
         Factors F;
         factors<VT, !BWD>(F, A, toff + col, valid);
         bad |= F.bad;
@@ -477,8 +488,8 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
         fB.put_t(c, l, F.B);
         fK.put_t(c, l, F.K);
         if constexpr (!BWD) {
-            fBh.put_t(c, l, F.Bh);
-            fKh.put_t(c, l, F.Kh);
+            Bh[i] = F.Bh;
+            Kh[i] = F.Kh;
         }
         if (l % 16 == 15) store4(ws + W::PL + col, F.P);
     }
@@ -511,11 +522,9 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
         for (int c = wave - 1; c < NB; c += 3) {
             if (!BWD) {
                 store4(ws + W::M1 + c * 256 + 4 * l, fR.t(c, l));
-                store4(ws + W::M2 + c * 256 + 4 * l, fBh.j(c, l));
-                store4(ws + W::M3 + c * 256 + 4 * l, fKh.j(c, l));
             } else {
-                store4(ws + W::M1 + c * 256 + 4 * l, fA.j(c, l));
-                store4(ws + W::M2 + c * 256 + 4 * l, fR.j(c, l));
+                store4(ws + W::M1 + c * 256 + 4 * l, fA.jp(c, l));
+                store4(ws + W::M2 + c * 256 + 4 * l, fR.jp(c, l));
             }
         }
         if (!BWD && wave >= 2) store_tile(ws + W::S + (wave - 1) * 256, l, m);
@@ -523,7 +532,20 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
         if (BWD && wave == 1) store_tile(ws + W::S + 512, l, m);
     }
     __syncthreads();
-    for (int c = wave; c < NB; c += 4) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int c = wave + 4 * i;
+        if (c >= NB) break;
+        if constexpr (!BWD) {
+            // B^ and K^ take the place of B~ and K~: a wave's own columns, to
+            // lanes of the other form (two matrices more in LDS halved the
+            // workgroups of a CU at N = 128, 66 -> 106 us)
+            fB.put_t(c, l, Bh[i]);
+            fK.put_t(c, l, Kh[i]);
+            __builtin_amdgcn_wave_barrier();
+            store4(ws + W::M2 + c * 256 + 4 * l, fB.jp(c, l));
+            store4(ws + W::M3 + c * 256 + 4 * l, fK.jp(c, l));
+        }
         const f4 wt =
             __builtin_convertvector(mm64(fA.jp(c, l), sM.dt(l)), f4);
         if (!BWD) {
@@ -577,7 +599,12 @@ __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
 // One wave per 16 state rows walks the segment's chunks with its rows of S
 // (or D) in registers; a workgroup's waves are row blocks of one head and
 // share each chunk's operands.  Bound by a wave's own chain of products: 19
-// of 16x16x16 a chunk forward at N = 64, 13 backward, 128 cycles each.
+// of 16x16x16 a chunk forward at N = 64, 13 backward, 128 cycles each, and the
+// update's eight (the state's, or its cotangent's) about 256: they are summed
+// in float64, onto the decayed state, and rounded once.  In float32 those sums
+// were the larger part of S_T's and dS0's error (0.7 and 0.9e-7 against 0.4
+// and 0.5), and under the slowest decay they added up to twice the sequential
+// kernels'.  At 32 chunks of 96 heads a chain takes 98 and 72 us for 77 and 59.
 template <int N>
 constexpr int kChainWaves = N / 16 < 4 ? N / 16 : 4;
 
@@ -783,20 +810,31 @@ f32_fwd_chain_kernel(Args A) {
         // the state
 #pragma unroll
         for (int c0 = 0; c0 < NB; c0 += G) {
-            f4 bk[2 * G], xv[2 * G], up[2 * G];
+            d4 acc[G];
+            f4 bb[G], kk[G];
 #pragma unroll
             for (int c = 0; c < G; ++c) {
-                bk[2 * c] = tile(W::M2 + (c0 + c) * 256);
-                bk[2 * c + 1] = tile(W::M3 + (c0 + c) * 256);
-                xv[2 * c] = x;
-                xv[2 * c + 1] = v;
+                bb[c] = tile(W::M2 + (c0 + c) * 256);
+                kk[c] = tile(W::M3 + (c0 + c) * 256);
+                acc[c] = __builtin_convertvector(s[c0 + c], d4) *
+                         __builtin_convertvector(
+                             load4(o + W::PL + 16 * (c0 + c) + 4 * q), d4);
             }
-            products(bk, xv, up);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < G; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        kk[c][e], v[e], acc[c], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < G; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        bb[c][e], x[e], acc[c], 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < G; ++c)
-                s[c0 + c] = s[c0 + c] *
-                                load4(o + W::PL + 16 * (c0 + c) + 4 * q) +
-                            (up[2 * c] + up[2 * c + 1]);
+                s[c0 + c] = __builtin_convertvector(acc[c], f4);
         }
         y += yx;
         // (the loads' values are taken before the stores are issued: memory
@@ -887,18 +925,29 @@ f32_bwd_chain_kernel(Args A) {
         }
 #pragma unroll
         for (int c0 = 0; c0 < NB; c0 += G) {
-            f4 ar[2 * G], uy[2 * G], up[2 * G];
+            d4 acc[G];
+            f4 aa[G], rr[G];
 #pragma unroll
             for (int c = 0; c < G; ++c) {
-                ar[2 * c] = tile(W::M1 + (c0 + c) * 256);
-                ar[2 * c + 1] = tile(W::M2 + (c0 + c) * 256);
-                uy[2 * c] = u;
-                uy[2 * c + 1] = dy;
+                aa[c] = tile(W::M1 + (c0 + c) * 256);
+                rr[c] = tile(W::M2 + (c0 + c) * 256);
+                acc[c] = __builtin_convertvector(d[c0 + c], d4);
             }
-            products(ar, uy, up);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < G; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        rr[c][e], dy[e], acc[c], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < G; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        aa[c][e], u[e], acc[c], 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < G; ++c)
-                d[c0 + c] += up[2 * c] + up[2 * c + 1];
+                d[c0 + c] = __builtin_convertvector(acc[c], f4);
         }
         feed.put(ops[buf == 0 ? 2 : buf - 1]);
         dy = yb.value();
