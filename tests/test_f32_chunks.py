@@ -222,3 +222,71 @@ def test_segment_of_one_partial_chunk(hip):
     torch.cuda.synchronize()
     for n, a, b in zip(GRADS, *outs):
         assert torch.equal(a, b), n
+
+
+@pytest.mark.parametrize("N,dtype,B,H,T", [(128, torch.bfloat16, 32, 32, 181),
+                                           (64, torch.float32, 30, 100, 150)])
+def test_time_segments(hip, N, dtype, B, H, T):
+    """Many heads: the workspace holds four chunks (N = 128, interval 32) or
+    three (N = 64) of 16 tokens forward and one backward, so the state, its
+    cotangent and the checkpoints pass from segment to segment.  Heads equal
+    the same heads in a call of few (one segment) bit for bit; three heads have
+    a chunk out of range, in the first, a middle and the last segment."""
+    tag = f"T{T} B{B} H{H} N{N} {dtype}"
+    print("case: chunked fp32, time segments", tag, flush=True)
+    x = make_inputs(T, B, H, N, dtype=dtype, seed=9, state_std=0.1,
+                    dstate_std=0.1, device="cuda", generator="torch")
+    nch = (T + 15) // 16
+    for h, ch in ((-1, 0), (-2, nch // 2), (-3, nch - 1)):
+        x["w"][16 * ch + 1:16 * ch + 4, -1, h] = 4.0
+    x["add"] = torch.randn(T, B, H, N, device="cuda").to(dtype)
+    states = ("s0", "ds_t", "s_t", "ds0")
+    x = {n: t if n in states else t.transpose(0, 1).contiguous()
+         for n, t in x.items()}
+
+    def last8(n, t):  # of the last batch row
+        return t[-1:, -8:] if n in states else t[:, -1:, -8:] if n == "ckpt" \
+            else t[-1:, :, -8:]
+
+    def in_range(n, t):
+        return t.narrow(1 if n in states else 2, 0, 5)
+
+    def run(x, ci):
+        vecs = [x[n] for n in (*NAMES, "s0")]
+        (y, s_t), aux = hip.forward_with_aux(*vecs, checkpoint_interval=ci,
+                                             layout="bthn")
+        assert hip.last_path() == "f32_forward"
+        out = {"y": y, "s_t": s_t, "ckpt": aux[0]}
+        if ci == 16:
+            g = hip.backward(*vecs, x["dy"], x["ds_t"], *aux, layout="bthn",
+                             add=(x["add"], None, x["add"]))
+            assert hip.last_path() == "f32_backward"
+            out.update(zip(GRADS, g))
+        return out
+
+    few = {n: last8(n, t).contiguous() for n, t in x.items()}
+    big = {}
+    for ci in (16, 32):
+        small = run(few, ci)
+        big[ci] = {n: last8(n, t).clone() for n, t in run(x, ci).items()}
+        torch.cuda.synchronize()
+        for n, t in big[ci].items():
+            assert torch.equal(in_range(n, t), in_range(n, small[n])), \
+                (tag, ci, n)
+    host = [_np(few[n]).swapaxes(0, 1) for n in NAMES]
+    host.append(_np(few["s0"]))
+    ey, es, eck = oracle.forward(*host, checkpoint_interval=16)
+    eg = list(oracle.backward(*host, _np(few["dy"]).swapaxes(0, 1),
+                              _np(few["ds_t"])))
+    want = {"s_t": es, "ckpt": eck, "ds0": eg[6]}
+    for n, e in (("y", ey), *zip(GRADS, eg[:6])):
+        want[n] = e.swapaxes(0, 1) + (_np(few["add"]) if n in ("dr", "dv")
+                                      else 0.0)
+    for n, e in want.items():
+        tol = 1e-4 if n in (*states, "ckpt") else TOL[dtype]
+        _close(n, big[16][n], e, tol, tag)
+    _close("y", big[32]["y"], want["y"], TOL[dtype], tag + " interval 32")
+    _close("s_t", big[32]["s_t"], es, 1e-4, tag + " interval 32")
+    # (the last entry is the final state)
+    eck = np.concatenate([eck[:-1:2], eck[-1:]])
+    _close("ckpt", big[32]["ckpt"], eck, 1e-4, tag + " interval 32")

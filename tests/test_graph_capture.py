@@ -48,9 +48,8 @@ def _replay_check(step, leaves, case):
 
 @pytest.mark.parametrize("n", [64, 128])
 def test_wkv7_operator_graph_replay(hip_lib, n):
-    # N = 128: the sequential kernels over row-split workgroups, whose
-    # partial column sums take stream-ordered memory from the library's pool
-    # (a memory node in the captured graph)
+    # N = 128: the chunked fp32 kernels, whose workspace is stream-ordered
+    # memory from the library's pool (a memory node in the captured graph)
     import rwkv7m_amd
     from rwkv7m_amd.kernels.wkv_ffi import unregister_wkv_ffi_backend
     print(f"case: wkv7 graph replay T70 B2 H2 N{n} bf16", flush=True)

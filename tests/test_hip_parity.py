@@ -122,7 +122,11 @@ def test_sequential_backward_saved_states_long_interval(hip, n):
     inp = make_inputs(300, 1, 2, n, dtype=torch.float32, seed=91,
                       state_std=0.1, dstate_std=0.1)
     ey, es, egrads = _oracle_all(inp)
-    y, s_t, aux, grads, _, _ = _run_hip(hip, _to_dev(inp), ci=256)
+    dev = _to_dev(inp)
+    y, s_t, aux, _, _, _ = _run_hip(hip, dev, ci=256)
+    grads = hip.backward(*(dev[n] for n in NAMES), dev["s0"], dev["dy"],
+                         dev["ds_t"], *aux)
+    assert hip.last_path() == "seq_backward"
     assert aux[0].shape[0] == 3
     _assert_close("y", y, ey, 1e-4, f"N={n}")
     _assert_close("s_t", s_t, es, 1e-4, f"N={n}")
@@ -134,13 +138,18 @@ def test_sequential_backward_row_split_time_segments(hip):
     """N = 128 splits each head's rows over two workgroups, whose shares of
     the column sums (dr, dw, dk, da, db) a second kernel adds; the shares of
     8 heads fit 3264 tokens at a time, so 3500 tokens run as two time
-    segments that pass dS through dS0."""
-    print("case: sequential backward, B2 T3500 H4 N128, interval 16",
+    segments that pass dS through dS0.  (An interval of 32: at 16 the chunked
+    fp32 kernels serve the backward.)"""
+    print("case: sequential backward, B2 T3500 H4 N128, interval 32",
           flush=True)
     inp = make_inputs(3500, 2, 4, 128, dtype=torch.float32, seed=93,
                       state_std=0.1, dstate_std=0.1)
     ey, es, egrads = _oracle_all(inp)
-    y, s_t, aux, grads, _, _ = _run_hip(hip, _to_dev(inp), ci=16)
+    dev = _to_dev(inp)
+    y, s_t, aux, _, _, _ = _run_hip(hip, dev, ci=32)
+    grads = hip.backward(*(dev[n] for n in NAMES), dev["s0"], dev["dy"],
+                         dev["ds_t"], *aux)
+    assert hip.last_path() == "seq_backward"
     _assert_close("y", y, ey, 1e-4, "N=128")
     _assert_close("s_t", s_t, es, 1e-4, "N=128")
     for name, g, e in zip(GRAD_NAMES, grads, egrads):

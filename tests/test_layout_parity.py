@@ -130,13 +130,19 @@ def test_chunked_batch_major_mixed_fallback(hip):
     (torch.bfloat16, 64, 3),
     (torch.bfloat16, 128, 16),
     (torch.float32, 128, 7),
+    (torch.float32, 64, 24),
+    (torch.bfloat16, 32, 24),
+    (torch.bfloat16, 128, 24),
 ])
 def test_sequential_batch_major_equals_time_major(hip, dtype, N, ci):
+    # (an interval of 16 at N >= 16 takes the chunked fp32 backward)
     case = f"sequential bthn T37 B2 H3 N{N} {dtype} ci{ci}"
     print("case:", case, flush=True)
     inp = make_inputs(37, 2, 3, N, dtype=dtype, seed=17 + N + ci,
                       state_std=0.1, dstate_std=0.1)
     tm, bm = _both_layouts(hip, inp, ci)
+    assert hip.last_path() == ("f32_backward" if ci == 16 else
+                               "seq_backward")
     _assert_identical(tm, bm, case)
     if dtype == torch.float32 and N in (64, 128):
         _check_oracle(bm, inp, ci, 1e-4, case)
