@@ -181,12 +181,19 @@ bool use_chunked(int dtype, int64_t N, int64_t ci, int64_t T,
 // bf16 ones with N = 16, 32 or 128, 16-byte aligned buffers, chunks whose
 // byte span stays below 2^31 and checkpoint intervals of whole chunks
 // (multiples of 16 up to 1024, which a time segment holds whole; 16
-// backward), from f32_min_tokens on: below that their three to five launches take longer than a sequential kernel's few tokens.
-// Measured as replayed graphs, 4 and 96 heads, chunked against sequential
-// (us): forward N = 64 T 64 29 / 22 and 31 / 23, T 128 36 / 41 and 43 / 43;
-// N = 32 T 192 34 / 38 and 39 / 39; N = 16 T 256 34 / 45 and 38 / 46; N = 128
-// T 64 41 / 49 and 53 / 52.  Backward N = 64 T 32 34 / 51 and 37 / 53; N = 16
-// T 32 28 / 22 and 29 / 22, T 48 28 / 31 and 30 / 31.
+// backward), from f32_min_tokens on: below that their three to five launches
+// take longer than a sequential kernel's few tokens.  Measured as replayed
+// graphs, fp32, 4 and 96 heads, chunked against sequential (us).
+//   forward   N = 16   T 192  32 / 33, 37 / 34   T 256  36 / 44, 45 / 45
+//             N = 32   T 128  31 / 27, 35 / 28   T 192  37 / 39, 46 / 40
+//             N = 64   T  64  30 / 22, 35 / 24   T 128  41 / 41, 49 / 44
+//             N = 128  T  32  34 / 26, 43 / 30   T  64  45 / 48, 57 / 52
+//   backward  N = 16   T  32  28 / 21, 27 / 22   T  48  27 / 31, 29 / 31
+//             N = 32   T  16  27 / 18, 28 / 19   T  32  29 / 32, 30 / 33
+//             N = 64   T  16  31 / 28, 33 / 30   T  32  34 / 51, 37 / 54
+//             N = 128  T  16  50 / 68, 59 / 79   T  32  55 / 118, 65 / 138
+// The forward's lines are where few heads break even; with many it does some
+// 64 tokens later (N = 64 T 192 64 / 65).
 int64_t f32_min_tokens(bool backward, int64_t N) {
     if (backward) return N == 16 ? 48 : 32;
     return N == 128 ? 64 : N == 64 ? 128 : N == 32 ? 192 : 256;
@@ -197,7 +204,8 @@ bool use_f32_chunks(int dtype, int64_t N, int64_t T, int64_t BH,
     if (N != 16 && N != 32 && N != 64 && N != 128) return false;
     if (dtype == RWKV7M_DTYPE_BF16 && N == 64) return false;
     if (token_stride * 64 >= (int64_t(1) << 31)) return false;
-    return T >= f32_min_tokens(backward, N) && BH <= (int64_t(1) << 22) && all_aligned16(ptrs);
+    return T >= f32_min_tokens(backward, N) && BH <= (int64_t(1) << 22) &&
+           all_aligned16(ptrs);
 }
 
 int forward_impl(const char* fn, int dtype, int64_t T, int64_t B, int64_t H,
