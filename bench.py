@@ -704,18 +704,16 @@ def bench_screening(args):
         tau_w = torch.tensor(0.1, device=dev)
         ages0 = torch.zeros(B, 16, device=dev)
         wargs = (base, st, se, kw, q, tau_w, mu, 0.05, 1e-6)
-        wout = screening_hip.write_scan(*wargs, state.slots, ages0)
-        wseq, ws32, wkeys = wout[0], wout[1], wout[-1]
+        wseq, ws32 = screening_hip.write(*wargs, state.slots, ages0)[:2]
         dwseq = torch.randn_like(wseq)
         btm = B * T * 16
         del calls["scan_fwd"], calls["scan_bwd"]
         calls["write_fwd"] = (
-            lambda: screening_hip.write_scan(*wargs, state.slots, ages0),
+            lambda: screening_hip.write(*wargs, state.slots, ages0),
             B * T * 128 * 2 + B * T * 64 * 4 + btm * 128 * (2 + 4)
             + btm * 16)
         calls["write_bwd"] = (
-            lambda: screening_hip.write_scan_backward(*wargs, ws32, wkeys,
-                                                      dwseq),
+            lambda: screening_hip.write_backward(*wargs, ws32, dwseq),
             B * T * 128 * 2 + B * T * 64 * 4 + btm * 128 * (4 + 2 + 4)
             + btm * 64 * 8 + btm * 4)
     kernels = {}

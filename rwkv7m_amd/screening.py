@@ -23,8 +23,9 @@ whole-sequence work:
 Steps 2 and 4 have HIP backward kernels; the rest is differentiated by
 torch autograd.  The read/write phase (``read_write`` with
 ``use_write_screening``) replaces step 2 with the write recurrence (HIP
-kernels ``rwkv7m_screen_write_scan`` and its backward), whose update strength
-depends on the slots' own write keys, and feeds the read per-step ages.
+kernels ``rwkv7m_screen_write_scan`` in fp32, ``rwkv7m_screen_write`` in bf16,
+and their backward), whose update strength depends on the slots' own write
+keys, and feeds the read per-step ages.
 Arithmetic follows the reference's dtypes: projections in the
 compute dtype, statistics, norms, the slots and the usage EMA in fp32.
 """
@@ -198,18 +199,23 @@ class _SlotProjection(torch.autograd.Function):
 
 
 class _WriteScan(torch.autograd.Function):
-    """The read/write phase's slot recurrence (HIP kernels
-    rwkv7m_screen_write_scan / _backward)."""
+    """The read/write phase's slot recurrence.  In fp32 with the write key
+    carried by its own recurrence (HIP kernels rwkv7m_screen_write_scan /
+    _backward: a training step at the 0.185B preset's slots takes 0.58 ms in
+    them where the projecting ones took 1.53).  In bf16 the key is the rounded
+    projection of the rounded slots, which does not follow a recurrence: the
+    kernels that project at every step (rwkv7m_screen_write / _backward)."""
 
     @staticmethod
     def forward(ctx, base, slot_term, slot_embed, kw, q_w, tau_w, mu,
                 slots0, ages0, floor, eps):
-        (seq, s32, ages_seq, rel_w, upd2, s_t, a_t,
-         keys) = screening_hip.write_scan(
+        carried = base.dtype == torch.float32
+        call = screening_hip.write_scan if carried else screening_hip.write
+        seq, s32, ages_seq, rel_w, upd2, s_t, a_t, *keys = call(
             base, slot_term, slot_embed, kw, q_w, tau_w, mu, floor, eps,
             slots0, ages0)
         ctx.save_for_backward(base, slot_term, slot_embed, kw, q_w, tau_w,
-                              mu, s32, keys)
+                              mu, s32, *keys)
         ctx.floor, ctx.eps = floor, eps
         ctx.mark_non_differentiable(upd2)
         ctx.set_materialize_grads(False)
@@ -217,17 +223,20 @@ class _WriteScan(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_seq, d_ages_seq, d_rel_w, _d_upd2, d_s_t, d_a_t):
-        (base, slot_term, slot_embed, kw, q_w, tau_w, mu, s32,
-         keys) = ctx.saved_tensors
+        base, slot_term, slot_embed, kw, q_w, tau_w, mu, s32, *keys = \
+            ctx.saved_tensors
         if d_seq is None:
             d_seq = torch.zeros(s32.shape, dtype=base.dtype,
                                 device=base.device)
-        (d_pre, d_s0, d_a0, d_emb, d_mu, d_keys, dq_w,
-         d_tau) = screening_hip.write_scan_backward(
+        call = (screening_hip.write_scan_backward if keys else
+                screening_hip.write_backward)
+        (d_pre, d_s0, d_a0, d_emb, d_mu, d_keys, dq_w, d_tau) = call(
             base, slot_term, slot_embed, kw, q_w, tau_w, mu, ctx.floor,
-            ctx.eps, s32, keys, d_seq, d_s_t, d_rel_w, d_ages_seq, d_a_t)
+            ctx.eps, s32, *keys, d_seq, d_s_t, d_rel_w, d_ages_seq, d_a_t)
+        if not keys:  # (per slot there)
+            dq_w = dq_w.sum(2)
         B, T, M, ds = s32.shape
-        skey = s32 + slot_embed.float()[None, None]
+        skey = (s32 + slot_embed.float()[None, None]).to(base.dtype).float()
         d_kw = torch.bmm(skey.reshape(B, -1, ds).transpose(1, 2).contiguous(),
                          d_keys.reshape(B, -1, kw.shape[1])).sum(0)
         return (d_pre.sum(2).to(base.dtype),

@@ -129,3 +129,49 @@ def test_an_empty_batch_is_refused(hip_lib):
     mod, x, h, _, state = _inputs(torch.float32, B=3, T=4, C=96)
     with pytest.raises(IndexError):
         mod(x[:0], h[:0], type(state)(*(t[:0] for t in state)))
+
+
+def _write_args(dtype, B=2, T=96, M=3, ds=80, dk=32, seed=4):
+    g = torch.Generator().manual_seed(seed)
+
+    def n(*shape):
+        return torch.randn(*shape, generator=g)
+
+    q = n(B, T, dk)
+    kw = (n(ds, dk) / ds ** 0.5).to(dtype)
+    return [t.cuda() for t in (
+        n(B, T, ds).to(dtype), 0.3 * n(M, ds), 0.5 * n(M, ds), kw,
+        q / q.norm(dim=-1, keepdim=True), torch.tensor(-0.6),
+        torch.full((M,), 0.02), 0.3 * n(B, M, ds),
+        torch.zeros(B, M))], 0.05, 1e-6
+
+
+def test_bf16_write_keys_are_rounded_projections(hip_lib):
+    """rel_w against the recurrence in float64 with the roundings of a bf16
+    projection, round(round(S + e) W): a rounding turned by the sums' order
+    moves single values, all others agree to fp32 (without the roundings all
+    are about 2^-9 off)."""
+    from rwkv7m_amd.screening import _WriteScan
+    print("case: screening write phase, bf16 keys", flush=True)
+    args, floor, eps = _write_args(torch.bfloat16)
+    _, _, rel_w, _, s_t, _ = _WriteScan.apply(*args, floor, eps)
+    torch.cuda.synchronize()
+    base, st, se, kw, q, tau, mu, S, _ = (t.double().cpu() for t in args)
+
+    def rnd(x):
+        return x.bfloat16().double()
+
+    want = []
+    for t in range(base.shape[1]):
+        k = rnd(rnd(S + se) @ kw)
+        sim = (k * q[:, t, None]).sum(-1) / torch.sqrt(
+            (k * k).sum(-1) + eps * eps)
+        rel = torch.clamp((sim - tau) / (1.0 - tau + eps), min=0.0) ** 2
+        want.append(rel)
+        rate = mu * torch.clamp(rel, min=floor)
+        S = S + rate[..., None] * (rnd(torch.tanh(base[:, t, None] + st)) - S)
+    want = torch.stack(want, 1)
+    err = (rel_w.double().cpu() - want).abs()
+    assert float(want.max()) > 0.1
+    assert float((err > 1e-5).double().mean()) < 0.05
+    assert float(err.max()) < 2.0 ** -7
