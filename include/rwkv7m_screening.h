@@ -154,43 +154,44 @@ int rwkv7m_screen_residual_backward(int pre_dtype, int h_dtype, int64_t n,
                                     void *stream);
 
 /*
- * The write phase in four passes around two products of the caller's, with
- * the write key carried by its own recurrence (the slots' update is linear,
- * and so is the key's projection):
- *   1. rwkv7m_screen_write_deltas: deltas [B][T][M][ds] = delta + slot_embed
- *      (fp32); the caller's product delta_keys = deltas kw.
+ * The write phase in fp32, with the write key carried by its own recurrence
+ * (the slots' update is linear, and so is the key's projection):
+ *   1. rwkv7m_screen_write_delta_keys: delta_keys [B][T][M][dk] =
+ *      (delta + slot_embed) kw;
  *   2. rwkv7m_screen_write_scan: as rwkv7m_screen_write, and keys
- *      [B][T][M][dk], the keys before normalisation (fp32, unrounded).
+ *      [B][T][M][dk], the keys before normalisation; keys may be delta_keys.
  * Backward:
- *   3. rwkv7m_screen_write_keys: p [B][T][M][dk] = (q - k^ sim) / |k| and
- *      sim [B][T][M]; the caller's product wp [B][T][M][ds] = p kw^T.
+ *   3. rwkv7m_screen_write_keys: p [B][T][M][dk] = (q - k^ sim) / |k|, sim
+ *      [B][T][M] and wp [B][T][M][ds] = p kw^T;
  *   4. rwkv7m_screen_write_scan_backward: as rwkv7m_screen_write_backward,
- *      with d_sim [B][T][M] in place of the keys' and queries' cotangents.
+ *      with d_sim [B][T][M] in place of the keys' and queries' cotangents;
  *   5. rwkv7m_screen_write_queries: p becomes d keys (times d_sim; d kw is
  *      the sum of (S_t + slot_embed)^T d keys), dq_w [B][T][dk].
  */
-int rwkv7m_screen_write_deltas(int dtype, int64_t B, int64_t T, int64_t M,
-                               int64_t ds, const void *base,
-                               const float *slot_term, const float *slot_embed,
-                               float *deltas, void *stream);
-int rwkv7m_screen_write_scan(int dtype, int64_t B, int64_t T, int64_t M,
-                             int64_t ds, int64_t dk, const void *base,
+int rwkv7m_screen_write_delta_keys(int64_t B, int64_t T, int64_t M, int64_t ds,
+                                   int64_t dk, const float *base,
+                                   const float *slot_term,
+                                   const float *slot_embed, const float *kw,
+                                   float *delta_keys, void *stream);
+int rwkv7m_screen_write_scan(int64_t B, int64_t T, int64_t M, int64_t ds,
+                             int64_t dk, const float *base,
                              const float *slot_term, const float *slot_embed,
                              const float *kw, const float *delta_keys,
                              const float *q_w, const float *tau_w,
                              const float *mu, double floor, double eps,
                              const float *slots0, const float *ages0,
-                             void *slots_seq, float *slots32, float *ages_seq,
+                             float *slots_seq, float *slots32, float *ages_seq,
                              float *rel_w, float *upd2, float *slots_T,
                              float *ages_T, float *keys, void *stream);
-int rwkv7m_screen_write_keys(int64_t B, int64_t T, int64_t M, int64_t dk,
-                             const float *keys, const float *q_w, double eps,
-                             float *p, float *sim, void *stream);
+int rwkv7m_screen_write_keys(int64_t B, int64_t T, int64_t M, int64_t ds,
+                             int64_t dk, const float *keys, const float *q_w,
+                             const float *kw, double eps, float *p, float *sim,
+                             float *wp, void *stream);
 int rwkv7m_screen_write_scan_backward(
-    int dtype, int64_t B, int64_t T, int64_t M, int64_t ds, const void *base,
+    int64_t B, int64_t T, int64_t M, int64_t ds, const float *base,
     const float *slot_term, const float *tau_w, const float *mu, double floor,
     double eps, const float *slots32, const float *sim, const float *wp,
-    const void *d_slots_seq, const float *d_slots_T, const float *d_rel_w,
+    const float *d_slots_seq, const float *d_slots_T, const float *d_rel_w,
     const float *d_ages_seq, const float *d_ages_T, float *d_pre,
     float *d_slots0, float *d_ages0, float *d_embed_part, float *d_mu_bm,
     float *d_sim, float *d_tau_w, void *stream);

@@ -6,9 +6,11 @@
 // S_{t+1} = S_t + s_t (delta_t - S_t), so
 //     K_{t+1} = K_t + s_t (D_t - K_t),   D_t = (delta_t + e) W,
 // with the D_t of all steps one product of [B T M, d_slot] by W before the
-// serial pass.  A step then holds two wave sums (|K|^2 and K . q) and no
-// matrix-vector product.  K runs in float64, so that what it loses against
-// the projection of the slots is the slots' own rounding.
+// serial pass.  A step then holds no matrix-vector product, only wave sums:
+// |K|^2 and K . q, which the next step waits for, and the update norm of each
+// 64 channels, which it does not.  K runs in float64, so that what it loses
+// against the projection of the slots is the slots' own rounding.  fp32 only:
+// with the slots and the key rounded to bf16 the key follows no recurrence.
 //
 // Backward: d K_t = dsim_t p_t with p_t = (q - k^ sim) / |K| known from the
 // forward, so its projection back to the slots is dsim_t (p_t W^T): again one
@@ -23,8 +25,10 @@
 //
 // Bound by the latency of a step.  At 128 slots x 512 steps of 128 channels,
 // keys of 64 (B = 8, M = 16), before (projecting kernels) -> now: forward
-// 570 -> 351 us, backward 958 -> 214 us, and 16 + 17 + 20 us in the passes
-// that form the deltas, the keys and the queries' cotangents.
+// 570 -> 338 us, backward 958 -> 214 us, and 44 + 18 + 43 + 19 us in the
+// passes that form the deltas' keys, the keys' cotangents and their
+// projection, and the queries'.  Those projections are this file's own kernels:
+// a library product would follow the caller's autocast and precision settings.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -43,10 +47,6 @@ constexpr int kBwdThreads = 64 * 9;  // the chain; four arrays x2
 __device__ __forceinline__ float wave_total(float x) {
     return add_swap<32>(add_swap<16>(group_sum<16>(x)));
 }
-__device__ __forceinline__ float rounded(float x, const float*) { return x; }
-__device__ __forceinline__ float rounded(float x, const bf16_t*) {
-    return bf16_to_f32(f32_to_bf16(x));
-}
 
 __device__ __forceinline__ int chunk_steps(int64_t ds, int dk) {
     const int n = kStage / int(ds > dk ? ds : dk);
@@ -56,8 +56,8 @@ __device__ __forceinline__ int chunk_steps(int64_t ds, int dk) {
 // Wave `part` of `parts` stages its batches of n rows of `width`, `stride`
 // elements apart, as fp32: 16 loads a lane in flight, from clamped in-bounds
 // addresses.
-template <typename E, typename F>
-__device__ __forceinline__ void stage(float* dst, const E* src, int64_t stride,
+template <typename F>
+__device__ __forceinline__ void stage(float* dst, const float* src, int64_t stride,
                                       int n, int width, F f, int part,
                                       int parts) {
     const int lane = threadIdx.x % 64, tot = n * width;
@@ -69,7 +69,7 @@ __device__ __forceinline__ void stage(float* dst, const E* src, int64_t stride,
             const int i = b0 + lane + 64 * r, ic = i < tot ? i : tot - 1;
             const int u = ic / width;
             col[r] = ic - u * width;
-            v[r] = load_f(src + u * stride + col[r]);
+            v[r] = src[u * stride + col[r]];
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -79,22 +79,121 @@ __device__ __forceinline__ void stage(float* dst, const E* src, int64_t stride,
     }
 }
 
-// delta_t + slot_embed for every step, the D_t product's left operand.
-template <typename E>
-__global__ __launch_bounds__(256) void write_deltas_kernel(ScreenScanWArgs A) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    const int64_t n = A.B * A.T * A.ds;
-    if (i >= n) return;
-    const int64_t row = i / A.ds, c = i - row * A.ds;
-    const E* base = static_cast<const E*>(A.base);
-    const float x = load_f(base + i);
-    for (int64_t m = 0; m < A.M; ++m)
-        A.deltas[(row * A.M + m) * A.ds + c] =
-            rounded(tanhf(x + A.slot_term[m * A.ds + c]), base) +
-            A.slot_embed[m * A.ds + c];
+// The two products around the scans: a wave takes H tiles of 16 rows
+// (b, t, m), its lane l (i = l % 16, q = l / 16) the operands of row i,
+// columns 4q .. 4q + 3 of each 16, and of the result's rows 4e + q, column i
+// of each 16.  Sums in float64 (v_mfma_f64_16x16x4_f64), rounded once.  At 65536
+// rows of 128, keys of 64, 44 and 43 us for 1.07 GFLOP each: above the matrix
+// core's 14 and the 50 MB's 10 by the loads' round trips.  (Two tiles a wave
+// for the first took 54, one for the second 71; a block's loads ahead of the
+// products of the block before 48 each.)
+using d4 = double __attribute__((ext_vector_type(4)));
+
+template <int H>
+struct ProductRows {
+    int64_t rows, row0;
+    int i, q;
+    __device__ __forceinline__ explicit ProductRows(const ScreenScanWArgs& A)
+        : rows(A.B * A.T * A.M),
+          row0((int64_t(blockIdx.x) * 4 + threadIdx.x / 64) * 16 * H),
+          i(threadIdx.x % 16),
+          q(threadIdx.x % 64 / 16) {}
+    // this lane's operand row of tile h (the last row past the end)
+    __device__ __forceinline__ int64_t in(int h) const {
+        const int64_t r = row0 + 16 * h + i;
+        return r < rows ? r : rows - 1;
+    }
+    __device__ __forceinline__ int64_t out(int h, int e) const {
+        return row0 + 16 * h + 4 * e + q;
+    }
+};
+
+// D_t = (delta_t + slot_embed) W for every step.
+template <int NJ>
+__global__ __launch_bounds__(256) void write_delta_keys_kernel(
+    ScreenScanWArgs A) {
+    const ProductRows<1> R(A);
+    if (R.row0 >= R.rows) return;
+    const int ds = int(A.ds), dk = A.dk;
+    const int64_t row = R.in(0), tok = row / A.M, m = row - tok * A.M;
+    const float* base = A.base + tok * ds;
+    const float* st = A.slot_term + m * ds;
+    const float* se = A.slot_embed + m * ds;
+    d4 acc[NJ] = {};
+    for (int c0 = 0; c0 < ds; c0 += 16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = c0 + 4 * R.q + e, cc = c < ds ? c : ds - 1;
+            const float x = tanhf(base[cc] + st[cc]) + se[cc];
+            const double a = c < ds ? double(x) : 0.0;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int col = 16 * j + R.i;
+                const float w = A.kw[cc * dk + (col < dk ? col : dk - 1)];
+                acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    a, c < ds ? double(w) : 0.0, acc[j], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t r = R.out(0, e);
+            if (r < R.rows && 16 * j + R.i < dk)
+                A.delta_keys_out[r * dk + 16 * j + R.i] = float(acc[j][e]);
+        }
 }
 
-template <typename E, int NCH>
+// wp = p W^T.
+template <int NJ>
+__global__ __launch_bounds__(256) void write_back_kernel(ScreenScanWArgs A) {
+    const ProductRows<2> R(A);
+    if (R.row0 >= R.rows) return;
+    const int ds = int(A.ds), dk = A.dk;
+    float x[2][NJ][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 16 * j + 4 * R.q + e;
+                x[h][j][e] = A.p[R.in(h) * dk + (k < dk ? k : dk - 1)];
+                x[h][j][e] = k < dk ? x[h][j][e] : 0.f;
+            }
+    for (int c0 = 0; c0 < ds; c0 += 16) {
+        const float* w = A.kw + (c0 + R.i < ds ? c0 + R.i : ds - 1) * dk;
+        float wv[NJ][4];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = 16 * j + 4 * R.q + e;
+                wv[j][e] = w[k < dk ? k : dk - 1];
+                wv[j][e] = k < dk ? wv[j][e] : 0.f;
+            }
+        d4 acc[2] = {};
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        double(x[h][j][e]), double(wv[j][e]), acc[h], 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int64_t r = R.out(h, e);
+                if (r < R.rows && c0 + R.i < ds)
+                    A.wp_out[r * ds + c0 + R.i] = float(acc[h][e]);
+            }
+    }
+}
+
+template <int NCH>
 __global__ __launch_bounds__(kFwdThreads) void write_scan_fwd_kernel(
     ScreenScanWArgs A) {
     __shared__ float sd[2][kStage], sq[2][kStage], sk[2][kStage];
@@ -104,9 +203,9 @@ __global__ __launch_bounds__(kFwdThreads) void write_scan_fwd_kernel(
     const int64_t b = blockIdx.x / A.M, m = blockIdx.x % A.M;
     const int64_t T = A.T, M = A.M, bm0 = b * T * M + m;
     const int ds = int(A.ds), dk = A.dk, ndw = (ds + 63) / 64;
-    const E* base = static_cast<const E*>(A.base) + b * T * ds;
+    const float* base = A.base + b * T * ds;
     const float* st = A.slot_term + m * ds;
-    E* seq = static_cast<E*>(A.slots_seq);
+    float* seq = A.slots_seq;
     const float mu = A.mu[m], tau = *A.tau_w, den = 1.f - tau + A.eps;
     const int chunk = chunk_steps(ds, dk);
     const int64_t nch = (T + chunk - 1) / chunk;
@@ -115,9 +214,9 @@ __global__ __launch_bounds__(kFwdThreads) void write_scan_fwd_kernel(
         const int n = int(T - t0 < chunk ? T - t0 : chunk), buf = int(ci & 1);
         const auto id = [](float x, int) { return x; };
         if (wave <= 2)
-            stage(sd[buf], base + t0 * ds, ds, n, ds, [&](float x, int c) {
-                return rounded(tanhf(x + st[c]), base);
-            }, wave - 1, 2);
+            stage(sd[buf], base + t0 * ds, ds, n, ds,
+                  [&](float x, int c) { return tanhf(x + st[c]); }, wave - 1,
+                  2);
         else if (wave == 3)
             stage(sq[buf], A.q_w + (b * T + t0) * dk, dk, n, dk, id, 0, 1);
         else
@@ -190,7 +289,7 @@ __global__ __launch_bounds__(kFwdThreads) void write_scan_fwd_kernel(
                     const int c = lane + 64 * i;
                     const bool in = c < ds;
                     if (in) {
-                        store_f(seq + row * ds + c, S[i]);
+                        seq[row * ds + c] = S[i];
                         A.slots32[row * ds + c] = S[i];
                     }
                     const float du = in ? s * (dl[i] - S[i]) : 0.f;
@@ -271,7 +370,7 @@ __global__ __launch_bounds__(256) void write_queries_kernel(
         if (lane + 64 * h < dk) A.dq_w[tok * dk + lane + 64 * h] = dq[h];
 }
 
-template <typename E, int NCH>
+template <int NCH>
 __global__ __launch_bounds__(kBwdThreads) void write_scan_bwd_kernel(
     ScreenScanWArgs A) {
     __shared__ float sth[2][kStage], ss[2][kStage], sg[2][kStage],
@@ -284,8 +383,8 @@ __global__ __launch_bounds__(kBwdThreads) void write_scan_bwd_kernel(
     const int64_t b = blockIdx.x / A.M, m = blockIdx.x % A.M;
     const int64_t T = A.T, M = A.M, bm0 = b * T * M + m;
     const int ds = int(A.ds);
-    const E* base = static_cast<const E*>(A.base) + b * T * ds;
-    const E* dseq = static_cast<const E*>(A.d_slots_seq) + bm0 * ds;
+    const float* base = A.base + b * T * ds;
+    const float* dseq = A.d_slots_seq + bm0 * ds;
     const float* st = A.slot_term + m * ds;
     const int64_t Mds = M * ds;
     const float mu = A.mu[m], tau = *A.tau_w, den = 1.f - tau + A.eps;
@@ -345,8 +444,7 @@ __global__ __launch_bounds__(kBwdThreads) void write_scan_bwd_kernel(
                     gv[i] = in ? sg[buf][u * ds + c] : 0.f;
                     wp[i] = in ? sp[buf][u * ds + c] : 0.f;
                     if (in)
-                        part += G[i] *
-                                (rounded(th[i], base) - ss[buf][u * ds + c]);
+                        part += G[i] * (th[i] - ss[buf][u * ds + c]);
                 }
                 const float dstr = wave_total(part);
                 const float drw = srel[buf][u] + (rw > A.floor ? dstr * mu : 0.f);
@@ -386,45 +484,44 @@ __global__ __launch_bounds__(kBwdThreads) void write_scan_bwd_kernel(
     }
 }
 
-template <typename E, int NCH>
+template <int NCH>
 void scan_n(bool backward, const ScreenScanWArgs& A, hipStream_t s) {
     const dim3 grid{unsigned(A.B * A.M)};
     if (backward)
-        hipLaunchKernelGGL((write_scan_bwd_kernel<E, NCH>), grid,
+        hipLaunchKernelGGL((write_scan_bwd_kernel<NCH>), grid,
                            dim3(kBwdThreads), 0, s, A);
     else
-        hipLaunchKernelGGL((write_scan_fwd_kernel<E, NCH>), grid,
+        hipLaunchKernelGGL((write_scan_fwd_kernel<NCH>), grid,
                            dim3(kFwdThreads), 0, s, A);
 }
 
-// Channels per lane: 2 and 4 at the presets (d_slot 128, 256).
-template <typename E>
-void scan(bool backward, const ScreenScanWArgs& A, hipStream_t s) {
-    if (A.ds <= 128)
-        scan_n<E, 2>(backward, A, s);
-    else if (A.ds <= 256)
-        scan_n<E, 4>(backward, A, s);
-    else
-        scan_n<E, 16>(backward, A, s);
+dim3 product_grid(const ScreenScanWArgs& A, int tiles) {
+    const int64_t rows = 64 * tiles;
+    return dim3(unsigned((A.B * A.T * A.M + rows - 1) / rows));
 }
 
 }  // namespace
 
-hipError_t launch_screen_write_deltas(bool bf16, const ScreenScanWArgs& A,
-                                      hipStream_t s) {
-    const dim3 grid(unsigned((A.B * A.T * A.ds + 255) / 256));
-    if (bf16)
-        hipLaunchKernelGGL(write_deltas_kernel<bf16_t>, grid, dim3(256), 0, s,
-                           A);
+hipError_t launch_screen_write_delta_keys(const ScreenScanWArgs& A,
+                                          hipStream_t s) {
+    if (A.dk <= 64)
+        hipLaunchKernelGGL((write_delta_keys_kernel<4>), product_grid(A, 1),
+                           dim3(256), 0, s, A);
     else
-        hipLaunchKernelGGL(write_deltas_kernel<float>, grid, dim3(256), 0, s,
-                           A);
+        hipLaunchKernelGGL((write_delta_keys_kernel<8>), product_grid(A, 1),
+                           dim3(256), 0, s, A);
     return hipGetLastError();
 }
 
-hipError_t launch_screen_write_scan(bool bf16, bool backward,
-                                    const ScreenScanWArgs& A, hipStream_t s) {
-    bf16 ? scan<bf16_t>(backward, A, s) : scan<float>(backward, A, s);
+// Channels per lane: 2 and 4 at the presets (d_slot 128, 256).
+hipError_t launch_screen_write_scan(bool backward, const ScreenScanWArgs& A,
+                                    hipStream_t s) {
+    if (A.ds <= 128)
+        scan_n<2>(backward, A, s);
+    else if (A.ds <= 256)
+        scan_n<4>(backward, A, s);
+    else
+        scan_n<16>(backward, A, s);
     return hipGetLastError();
 }
 
@@ -432,6 +529,12 @@ hipError_t launch_screen_write_keys(const ScreenScanWArgs& A, hipStream_t s) {
     hipLaunchKernelGGL(write_keys_kernel,
                        dim3(unsigned((A.B * A.T * A.M + 3) / 4)), dim3(256), 0,
                        s, A);
+    if (A.dk <= 64)
+        hipLaunchKernelGGL((write_back_kernel<4>), product_grid(A, 2), dim3(256),
+                           0, s, A);
+    else
+        hipLaunchKernelGGL((write_back_kernel<8>), product_grid(A, 2), dim3(256),
+                           0, s, A);
     return hipGetLastError();
 }
 

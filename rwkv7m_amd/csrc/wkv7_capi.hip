@@ -1134,44 +1134,49 @@ int rwkv7m_screen_slot_scan_backward(
                           static_cast<hipStream_t>(stream)));
 }
 
-int rwkv7m_screen_write_deltas(int dtype, int64_t B, int64_t T, int64_t M,
-                               int64_t ds, const void* base,
-                               const float* slot_term, const float* slot_embed,
-                               float* deltas, void* stream) {
-    const char* fn = "rwkv7m_screen_write_deltas";
+int rwkv7m_screen_write_delta_keys(int64_t B, int64_t T, int64_t M, int64_t ds,
+                                   int64_t dk, const float* base,
+                                   const float* slot_term,
+                                   const float* slot_embed, const float* kw,
+                                   float* delta_keys, void* stream) {
+    const char* fn = "rwkv7m_screen_write_delta_keys";
     g_last_error.clear();
-    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, 1, 0.0, 0.0));
-    if (B == 0 || T == 0 || M == 0 || ds == 0) return RWKV7M_OK;
+    RWKV7M_TRY(
+        sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, ds, dk, 0.0, 0.0));
+    if (B == 0 || T == 0 || M == 0) return RWKV7M_OK;
     RWKV7M_TRY(sc_need(fn, {{"base", base}, {"slot_term", slot_term},
-                            {"slot_embed", slot_embed}, {"deltas", deltas}}));
+                            {"slot_embed", slot_embed}, {"kw", kw},
+                            {"delta_keys", delta_keys}}));
     rwkv7m::ScreenScanWArgs A{};
     A.B = B;
     A.T = T;
     A.M = M;
     A.ds = ds;
+    A.dk = int(dk);
     A.base = base;
     A.slot_term = slot_term;
     A.slot_embed = slot_embed;
-    A.deltas = deltas;
-    return hip_status("screening write deltas launch",
-                      rwkv7m::launch_screen_write_deltas(
-                          dtype == RWKV7M_DTYPE_BF16, A,
-                          static_cast<hipStream_t>(stream)));
+    A.kw = kw;
+    A.delta_keys_out = delta_keys;
+    return hip_status("screening write delta keys launch",
+                      rwkv7m::launch_screen_write_delta_keys(
+                          A, static_cast<hipStream_t>(stream)));
 }
 
-int rwkv7m_screen_write_scan(int dtype, int64_t B, int64_t T, int64_t M,
-                             int64_t ds, int64_t dk, const void* base,
+int rwkv7m_screen_write_scan(int64_t B, int64_t T, int64_t M, int64_t ds,
+                             int64_t dk, const float* base,
                              const float* slot_term, const float* slot_embed,
                              const float* kw, const float* delta_keys,
                              const float* q_w, const float* tau_w,
                              const float* mu, double floor, double eps,
                              const float* slots0, const float* ages0,
-                             void* slots_seq, float* slots32, float* ages_seq,
+                             float* slots_seq, float* slots32, float* ages_seq,
                              float* rel_w, float* upd2, float* slots_T,
                              float* ages_T, float* keys, void* stream) {
     const char* fn = "rwkv7m_screen_write_scan";
     g_last_error.clear();
-    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, dk, floor, eps));
+    RWKV7M_TRY(
+        sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, ds, dk, floor, eps));
     if (B == 0 || M == 0 || ds == 0) return RWKV7M_OK;
     RWKV7M_TRY(sc_need(fn, {{"slot_term", slot_term},
                             {"slot_embed", slot_embed}, {"kw", kw},
@@ -1212,45 +1217,50 @@ int rwkv7m_screen_write_scan(int dtype, int64_t B, int64_t T, int64_t M,
     A.keys = keys;
     return hip_status("screening write scan launch",
                       rwkv7m::launch_screen_write_scan(
-                          dtype == RWKV7M_DTYPE_BF16, false, A,
-                          static_cast<hipStream_t>(stream)));
+                          false, A, static_cast<hipStream_t>(stream)));
 }
 
-int rwkv7m_screen_write_keys(int64_t B, int64_t T, int64_t M, int64_t dk,
-                             const float* keys, const float* q_w, double eps,
-                             float* p, float* sim, void* stream) {
+int rwkv7m_screen_write_keys(int64_t B, int64_t T, int64_t M, int64_t ds,
+                             int64_t dk, const float* keys, const float* q_w,
+                             const float* kw, double eps, float* p, float* sim,
+                             float* wp, void* stream) {
     const char* fn = "rwkv7m_screen_write_keys";
     g_last_error.clear();
-    RWKV7M_TRY(sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, 1, dk, 0.0, eps));
+    RWKV7M_TRY(
+        sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, ds, dk, 0.0, eps));
     if (B == 0 || T == 0 || M == 0) return RWKV7M_OK;
-    RWKV7M_TRY(sc_need(fn, {{"keys", keys}, {"q_w", q_w}, {"p", p},
-                            {"sim", sim}}));
+    RWKV7M_TRY(sc_need(fn, {{"keys", keys}, {"q_w", q_w}, {"kw", kw}, {"p", p},
+                            {"sim", sim}, {"wp", wp}}));
     rwkv7m::ScreenScanWArgs A{};
     A.B = B;
     A.T = T;
     A.M = M;
     A.dk = int(dk);
     A.eps = float(eps);
+    A.ds = ds;
     A.keys = const_cast<float*>(keys);
     A.q_w = q_w;
+    A.kw = kw;
     A.p = p;
     A.sim = sim;
+    A.wp_out = wp;
     return hip_status("screening write keys launch",
                       rwkv7m::launch_screen_write_keys(
                           A, static_cast<hipStream_t>(stream)));
 }
 
 int rwkv7m_screen_write_scan_backward(
-    int dtype, int64_t B, int64_t T, int64_t M, int64_t ds, const void* base,
+    int64_t B, int64_t T, int64_t M, int64_t ds, const float* base,
     const float* slot_term, const float* tau_w, const float* mu, double floor,
     double eps, const float* slots32, const float* sim, const float* wp,
-    const void* d_slots_seq, const float* d_slots_T, const float* d_rel_w,
+    const float* d_slots_seq, const float* d_slots_T, const float* d_rel_w,
     const float* d_ages_seq, const float* d_ages_T, float* d_pre,
     float* d_slots0, float* d_ages0, float* d_embed_part, float* d_mu_bm,
     float* d_sim, float* d_tau_w, void* stream) {
     const char* fn = "rwkv7m_screen_write_scan_backward";
     g_last_error.clear();
-    RWKV7M_TRY(sc_write_checks(fn, dtype, B, T, M, ds, 1, floor, eps));
+    RWKV7M_TRY(
+        sc_write_checks(fn, RWKV7M_DTYPE_F32, B, T, M, ds, 1, floor, eps));
     if (B == 0 || M == 0 || ds == 0) return RWKV7M_OK;
     RWKV7M_TRY(sc_need(fn, {{"slot_term", slot_term}, {"tau_w", tau_w},
                             {"mu", mu}, {"d_slots0", d_slots0},
@@ -1291,8 +1301,7 @@ int rwkv7m_screen_write_scan_backward(
     A.d_tau_w = d_tau_w;
     return hip_status("screening write scan backward launch",
                       rwkv7m::launch_screen_write_scan(
-                          dtype == RWKV7M_DTYPE_BF16, true, A,
-                          static_cast<hipStream_t>(stream)));
+                          true, A, static_cast<hipStream_t>(stream)));
 }
 
 int rwkv7m_screen_write_queries(int64_t B, int64_t T, int64_t M, int64_t dk,

@@ -259,24 +259,23 @@ struct ScreenScanWArgs {
     int64_t B, T, M, ds;
     int dk;
     float floor, eps;
-    const void* base;                          // [B][T][ds]
+    const float* base;                         // [B][T][ds]
     const float *slot_term, *slot_embed, *kw;  // [M][ds] x2, [ds][dk]
     const float *delta_keys, *q_w;             // [B][T][M][dk], [B][T][dk]
     const float *tau_w, *mu, *slots0, *ages0;
-    float* deltas;                             // [B][T][M][ds]
-    void* slots_seq;
+    float *delta_keys_out, *wp_out;            // [B][T][M][dk], [B][T][M][ds]
+    float* slots_seq;
     float *slots32, *ages_seq, *rel_w, *upd2, *slots_T, *ages_T;
     float *keys, *p, *sim;                     // [B][T][M][dk] x2, [B][T][M]
     const float* wp;                           // [B][T][M][ds]
-    const void* d_slots_seq;
+    const float* d_slots_seq;
     const float *d_slots_T, *d_rel_w, *d_ages_seq, *d_ages_T;  // may be 0
     float *d_pre, *d_slots0, *d_ages0, *d_embed_part, *d_mu_bm, *d_sim,
         *d_tau_w, *dq_w;
 };
-hipError_t launch_screen_write_deltas(bool bf16, const ScreenScanWArgs& A,
-                                      hipStream_t stream);
-hipError_t launch_screen_write_scan(bool bf16, bool backward,
-                                    const ScreenScanWArgs& A,
+hipError_t launch_screen_write_delta_keys(const ScreenScanWArgs& A,
+                                          hipStream_t stream);
+hipError_t launch_screen_write_scan(bool backward, const ScreenScanWArgs& A,
                                     hipStream_t stream);
 hipError_t launch_screen_write_keys(const ScreenScanWArgs& A,
                                     hipStream_t stream);

@@ -306,8 +306,11 @@ def stats(rel, rel_w, z_norm, u_norm, upd2, usage0, floor, decay):
 
 def write_scan(base, slot_term, slot_embed, kw, q_w, tau_w, mu, floor, eps,
                slots0, ages0):
-    """``write`` with the write key carried by its own recurrence: the same
-    outputs, and the keys [B, T, M, dk] (fp32) for ``write_scan_backward``."""
+    """``write`` in fp32 with the write key carried by its own recurrence:
+    the same outputs, and the keys [B, T, M, dk] for
+    ``write_scan_backward``."""
+    if base.dtype != torch.float32:
+        raise TypeError(f"write_scan takes a float32 base, got {base.dtype}")
     base, st, se, kw_, qw, tw, mu_ = _write_common(base, slot_term,
                                                    slot_embed, kw, q_w, tau_w,
                                                    mu)
@@ -316,22 +319,19 @@ def write_scan(base, slot_term, slot_embed, kw, q_w, tau_w, mu, floor, eps,
     dev = _check([("base", base, (B, T, ds)), ("slots0", slots0, (B, M, ds)),
                   ("ages0", ages0, (B, M))])
     f = dict(dtype=torch.float32, device=dev)
-    P, code = wkv_hip._p, wkv_hip._dtype_code(base)
-    deltas = torch.empty(B, T, M, ds, **f)
-    _call("rwkv7m_screen_write_deltas", code, B, T, M, ds, P(base), P(st),
-          P(se), P(deltas), wkv_hip._stream(dev))
-    delta_keys = deltas @ kw_
-    seq = torch.empty(B, T, M, ds, dtype=base.dtype, device=dev)
-    s32 = deltas  # (its buffer: the products above are queued before)
+    P, strm = wkv_hip._p, wkv_hip._stream(dev)
+    keys = torch.empty(B, T, M, dk, **f)  # (the deltas' first)
+    _call("rwkv7m_screen_write_delta_keys", B, T, M, ds, dk, P(base), P(st),
+          P(se), P(kw_), P(keys), strm)
+    seq, s32 = torch.empty(B, T, M, ds, **f), torch.empty(B, T, M, ds, **f)
     ages_seq, rel_w = torch.empty(B, T, M, **f), torch.empty(B, T, M, **f)
     upd2 = torch.empty(B, T, M, (ds + 63) // 64, **f)
     s_t, a_t = torch.empty(B, M, ds, **f), torch.empty(B, M, **f)
-    keys = torch.empty(B, T, M, dk, **f)
     s0, a0 = _f32(slots0), _f32(ages0)
-    _call("rwkv7m_screen_write_scan", code, B, T, M, ds, dk, P(base), P(st),
-          P(se), P(kw_), P(delta_keys), P(qw), P(tw), P(mu_), float(floor),
-          float(eps), P(s0), P(a0), P(seq), P(s32), P(ages_seq), P(rel_w),
-          P(upd2), P(s_t), P(a_t), P(keys), wkv_hip._stream(dev))
+    _call("rwkv7m_screen_write_scan", B, T, M, ds, dk, P(base), P(st), P(se),
+          P(kw_), P(keys), P(qw), P(tw), P(mu_), float(floor), float(eps),
+          P(s0), P(a0), P(seq), P(s32), P(ages_seq), P(rel_w), P(upd2),
+          P(s_t), P(a_t), P(keys), strm)
     return seq, s32, ages_seq, rel_w, upd2, s_t, a_t, keys
 
 
@@ -361,17 +361,16 @@ def write_scan_backward(base, slot_term, slot_embed, kw, q_w, tau_w, mu,
     d_seq = _c(d_slots_seq).to(base.dtype)
     cots = [_f32(t) for t in (d_slots_T, d_rel_w, d_ages_seq, d_ages_T)]
     p, sim = torch.empty(B, T, M, dk, **f), torch.empty(B, T, M, **f)
-    _call("rwkv7m_screen_write_keys", B, T, M, dk, P(keys), P(qw), float(eps),
-          P(p), P(sim), strm)
-    wp = p @ kw_.t()
+    wp = torch.empty(B, T, M, ds, **f)
+    _call("rwkv7m_screen_write_keys", B, T, M, ds, dk, P(keys), P(qw), P(kw_),
+          float(eps), P(p), P(sim), P(wp), strm)
     outs = [torch.empty(B, T, M, ds, **f), torch.empty(B, M, ds, **f),
             torch.empty(B, M, **f), torch.empty(B, M, ds, **f),
             torch.empty(B, M, **f)]
     d_sim, d_tau = torch.empty(B, T, M, **f), torch.empty(B, T, M, **f)
-    _call("rwkv7m_screen_write_scan_backward", wkv_hip._dtype_code(base), B,
-          T, M, ds, P(base), P(st), P(tw), P(mu_), float(floor), float(eps),
-          P(s32), P(sim), P(wp), P(d_seq), *map(P, cots), *map(P, outs),
-          P(d_sim), P(d_tau), strm)
+    _call("rwkv7m_screen_write_scan_backward", B, T, M, ds, P(base), P(st),
+          P(tw), P(mu_), float(floor), float(eps), P(s32), P(sim), P(wp),
+          P(d_seq), *map(P, cots), *map(P, outs), P(d_sim), P(d_tau), strm)
     dq = torch.empty(B, T, dk, **f)
     _call("rwkv7m_screen_write_queries", B, T, M, dk, P(keys), P(d_sim),
           float(eps), P(p), P(dq), strm)

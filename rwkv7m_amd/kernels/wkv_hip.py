@@ -84,7 +84,7 @@ EXPORTED_SYMBOLS = (
     "rwkv7m_screen_residual",
     "rwkv7m_screen_residual_backward",
     "rwkv7m_screen_stats",
-    "rwkv7m_screen_write_deltas",
+    "rwkv7m_screen_write_delta_keys",
     "rwkv7m_screen_write_scan",
     "rwkv7m_screen_write_keys",
     "rwkv7m_screen_write_scan_backward",
@@ -188,11 +188,11 @@ def load_library(path: str | None = None):
         for name, args in (
                 ("residual", [i32] * 2 + [i64] + [vp] * 6),
                 ("residual_backward", [i32] * 2 + [i64] + [vp] * 8),
-                ("write_deltas", [i32] + [i64] * 4 + [vp] * 5),
-                ("write_scan", [i32] + [i64] * 5 + [vp] * 8 + [f64] * 2 +
+                ("write_delta_keys", [i64] * 5 + [vp] * 6),
+                ("write_scan", [i64] * 5 + [vp] * 8 + [f64] * 2 +
                  [vp] * 11),
-                ("write_keys", [i64] * 4 + [vp] * 2 + [f64] + [vp] * 3),
-                ("write_scan_backward", [i32] + [i64] * 4 + [vp] * 4 +
+                ("write_keys", [i64] * 5 + [vp] * 3 + [f64] + [vp] * 4),
+                ("write_scan_backward", [i64] * 4 + [vp] * 4 +
                  [f64] * 2 + [vp] * 16),
                 ("write_queries", [i64] * 4 + [vp] * 2 + [f64] + [vp] * 3),
                 ("stats", [i64] * 4 + [vp] * 6 + [f64] * 2 + [vp] * 4)):

@@ -201,7 +201,7 @@ class _SlotProjection(torch.autograd.Function):
 class _WriteScan(torch.autograd.Function):
     """The read/write phase's slot recurrence.  In fp32 with the write key
     carried by its own recurrence (HIP kernels rwkv7m_screen_write_scan /
-    _backward: a training step at the 0.185B preset's slots takes 0.58 ms in
+    _backward: a training step at the 0.185B preset's slots takes 0.67 ms in
     them where the projecting ones took 1.53).  In bf16 the key is the rounded
     projection of the rounded slots, which does not follow a recurrence: the
     kernels that project at every step (rwkv7m_screen_write / _backward)."""

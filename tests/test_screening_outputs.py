@@ -175,3 +175,58 @@ def test_bf16_write_keys_are_rounded_projections(hip_lib):
     assert float(want.max()) > 0.1
     assert float((err > 1e-5).double().mean()) < 0.05
     assert float(err.max()) < 2.0 ** -7
+
+
+def test_write_phase_under_autocast(hip_lib):
+    """The keys are the kernels' own fp32 products: an autocast region does
+    not turn them into bf16 ones."""
+    from rwkv7m_amd.screening import _WriteScan
+    print("case: screening write phase under autocast", flush=True)
+    args, floor, eps = _write_args(torch.float32)
+    res = []
+    for on in (False, True):
+        leaves = [t.clone().requires_grad_() for t in args]
+        with torch.autocast("cuda", torch.bfloat16, enabled=on):
+            out = _WriteScan.apply(*leaves, floor, eps)
+            diff = [out[0], out[2], out[4]]
+            grads = torch.autograd.grad(
+                [t.float().square().sum() for t in diff],
+                leaves[:3] + leaves[4:8])
+        res.append([*out, *grads])
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(*res)):
+        assert torch.isfinite(a).all() and torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("B,T,M,ds,dk", [(1, 1, 1, 1, 1), (1, 5, 3, 17, 15),
+                                         (2, 8, 4, 16, 16), (1, 13, 5, 33, 64),
+                                         (1, 3, 7, 130, 65),
+                                         (2, 9, 2, 300, 128)])
+def test_write_products(hip_lib, B, T, M, ds, dk):
+    """delta_keys and wp at the edges of their 16-row, 16-column tiles, against
+    float64: one rounding and tanh's few ulps, 1e-6 of the terms' size."""
+    from rwkv7m_amd.kernels import screening_hip as sh
+    from rwkv7m_amd.kernels import wkv_hip
+    print("case: screening write products", B, T, M, ds, dk, flush=True)
+    g = torch.Generator("cuda").manual_seed(ds + dk)
+
+    def n(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+
+    base, st, se, kw = n(B, T, ds), n(M, ds), n(M, ds), n(ds, dk)
+    keys, q = n(B, T, M, dk), n(B, T, dk)
+    dkeys, p, wp = (torch.full((B, T, M, k), float("nan"), device="cuda")
+                    for k in (dk, dk, ds))
+    sim = torch.empty(B, T, M, device="cuda")
+    P, strm = wkv_hip._p, wkv_hip._stream(base.device)
+    sh._call("rwkv7m_screen_write_delta_keys", B, T, M, ds, dk, P(base), P(st),
+             P(se), P(kw), P(dkeys), strm)
+    sh._call("rwkv7m_screen_write_keys", B, T, M, ds, dk, P(keys), P(q), P(kw),
+             1e-6, P(p), P(sim), P(wp), strm)
+    x = torch.tanh(base.double()[:, :, None] + st.double()) + se.double()
+    for got, a, w in ((dkeys, x, kw.double()), (wp, p.double(),
+                                                kw.double().t())):
+        a, w = a.cpu(), w.cpu()
+        err = (got.double().cpu() - a @ w).abs()
+        assert (err <= 1e-6 * (a.abs() @ w.abs()) + 1e-30).all(), \
+            float(err.max())
