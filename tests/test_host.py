@@ -520,6 +520,35 @@ def test_screening_write_abi_checks_requests_before_any_device_call(lib):
     assert b"d_pre is NULL" in lib.rwkv7m_last_error()
 
 
+def test_carried_write_keys_abi_checks_requests_before_any_device_call(lib):
+    fake = 1 << 20
+    dims = (2, 8, 4, 128, 64)  # B, T, M, ds, dk
+    dkeys = lib.rwkv7m_screen_write_delta_keys
+    assert dkeys(2, 8, 4, 128, 200, *([fake] * 5), None) == 2
+    assert b"dk <= 128" in lib.rwkv7m_last_error()
+    assert dkeys(*dims, *([fake] * 4), None, None) == 1
+    assert b"delta_keys is NULL" in lib.rwkv7m_last_error()
+    assert dkeys(0, 8, 4, 128, 64, *([None] * 5), None) == 0
+    scan = lib.rwkv7m_screen_write_scan
+    assert scan(*dims, *([fake] * 8), 0.05, 1e-6, *([fake] * 9), None,
+                None) == 1
+    assert b"keys is NULL" in lib.rwkv7m_last_error()
+    keys = lib.rwkv7m_screen_write_keys
+    assert keys(*dims, fake, fake, None, 1e-6, *([fake] * 3), None) == 1
+    assert b"kw is NULL" in lib.rwkv7m_last_error()
+    assert keys(*dims, *([fake] * 3), -1.0, *([fake] * 3), None) == 1
+    assert b"floor and eps" in lib.rwkv7m_last_error()
+    res = lib.rwkv7m_screen_residual
+    assert res(3, 1, 8, *([fake] * 5), None) == 1
+    assert b"bfloat16 or float32" in lib.rwkv7m_last_error()
+    assert res(1, 1, -8, *([fake] * 5), None) == 1
+    assert b"negative size" in lib.rwkv7m_last_error()
+    bwd = lib.rwkv7m_screen_residual_backward
+    assert bwd(0, 1, 8, *([fake] * 6), None, None) == 1
+    assert b"d_lam is NULL" in lib.rwkv7m_last_error()
+    assert bwd(0, 1, 0, *([None] * 7), None) == 0
+
+
 def test_screening_config_checks_follow_the_reference():
     """ScreeningConfig.__post_init__ rejects what the reference's does, with
     its messages (src/rwkv7m/model/screening.py:124-140), and the module's

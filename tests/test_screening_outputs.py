@@ -230,3 +230,34 @@ def test_write_products(hip_lib, B, T, M, ds, dk):
         err = (got.double().cpu() - a @ w).abs()
         assert (err <= 1e-6 * (a.abs() @ w.abs()) + 1e-30).all(), \
             float(err.max())
+
+
+@pytest.mark.parametrize("T,M,ds,dk", [(70, 3, 128, 64), (30, 2, 300, 30),
+                                       (20, 2, 260, 72), (20, 3, 256, 64)])
+def test_projecting_and_carried_write_keys_agree(hip_lib, T, M, ds, dk):
+    """rwkv7m_screen_write (the key projected at every step) in fp32, for
+    callers of the C interface, against the carried key's kernels: forward and
+    every cotangent, to 1e-5 of the largest (sums of up to 300 terms and T
+    steps of 2^-24 each)."""
+    from rwkv7m_amd.kernels import screening_hip as sh
+    print("case: screening write keys", T, M, ds, dk, flush=True)
+    (base, st, se, kw, q, tau, mu, s0, a0), floor, eps = _write_args(
+        torch.float32, T=T, M=M, ds=ds, dk=dk)
+    args = (base, st, se, kw, q, tau, mu, floor, eps)
+    want = sh.write(*args, s0, a0)
+    *got, keys = sh.write_scan(*args, s0, a0)
+    g = torch.Generator("cuda").manual_seed(6)
+    cots = [torch.randn(t.shape, generator=g, device="cuda")
+            for t in (want[0], want[5], want[3], want[2], want[6])]
+    wb = list(sh.write_backward(*args, want[1], *cots))
+    gb = list(sh.write_scan_backward(*args, got[1], keys, *cots))
+    wb[6] = wb[6].sum(2)
+    torch.cuda.synchronize()
+    assert torch.equal(got[2], want[2])  # ages
+    assert float(want[3].max()) > floor  # the relevance is in play
+    for n, a, b in zip(("seq", "s32", "ages", "rel_w", "upd2", "s_t", "a_t",
+                        "d_pre", "d_slots0", "d_ages0", "d_embed", "d_mu",
+                        "d_keys", "dq_w", "d_tau"), (*got, *gb),
+                       (*want, *wb)):
+        err = float((a - b).abs().max()) / (float(b.abs().max()) or 1.0)
+        assert err <= 1e-5, (n, err)
