@@ -34,8 +34,9 @@
  * rwkv7m_status and rwkv7m_last_error() describes it (thread-local).
  * Supported head sizes N: 1, 2, 4, 8, 16, 32, 64, 128.  The MFMA chunked
  * kernels serve bf16 with N == 64; fp32 with N == 16, 32, 64 or 128 and bf16
- * with N == 16, 32 or 128 run chunked fp32 kernels from a few dozen tokens
- * on, whose workspace (200 MB, or one checkpoint interval forward and one
+ * with N == 16, 32 or 128 run chunked fp32 kernels from a few dozen tokens on
+ * (a few hundred in the forward, which up to N == 64 also takes at most a head
+ * a CU), whose workspace (200 MB, or one checkpoint interval forward and one
  * chunk of 16 tokens backward of all heads where that is more, up to 37 and
  * 110 KB a chunk and head) comes from a stream-ordered pool;
  * every other case, and a call whose workspace does not fit, runs the

@@ -192,10 +192,23 @@ bool use_chunked(int dtype, int64_t N, int64_t ci, int64_t T,
 //             N = 32   T  16  27 / 18, 28 / 19   T  32  29 / 32, 30 / 33
 //             N = 64   T  16  31 / 28, 33 / 30   T  32  34 / 51, 37 / 54
 //             N = 128  T  16  50 / 68, 59 / 79   T  32  55 / 118, 65 / 138
-// The forward's lines are where few heads break even; with many it does some
-// 64 tokens later (N = 64 T 192 64 / 65).
-int64_t f32_min_tokens(bool backward, int64_t N) {
+// The forward breaks even later with many heads, past a quarter of the CUs (96
+// heads: N = 16 T 320 52 / 56, N = 32 T 256 55 / 52, N = 64 T 192 64 / 65, N =
+// 128 T 96 69 / 77).  Up to N = 64 the forward also needs
+// at most one head a CU: past that the sequential kernel fills the chip with
+// its heads, and the chunked kernels' passes over the workspace cost more than
+// its tokens.  Without and with checkpoints, T 512, chunked against sequential:
+//   N = 16    128 heads  74 / 92, 75 / 101     256   96 / 94, 94 / 101
+//             512       137 / 96, 135 / 106   1024  268 / 116, 272 / 126
+//   N = 32    128        94 / 108, 95 / 117    256  123 / 111, 121 / 118
+//             512       212 / 139, 213 / 162  1024  354 / 246, 378 / 257
+//   N = 64    128       135 / 164, 144 / 178   256  185 / 187, 209 / 207
+//             512       332 / 287, 373 / 329  1024  695 / 589, 764 / 656
+//   N = 128   256       538 / 748, 626 / 794  1024  2419 / 2965, 2723 / 3143
+// The backward wins at all of them (N = 16, 1024 heads 520 / 663).
+int64_t f32_min_tokens(bool backward, int64_t N, bool many_heads) {
     if (backward) return N == 16 ? 48 : 32;
+    if (many_heads) return N == 128 ? 96 : N == 64 ? 192 : 320;
     return N == 128 ? 64 : N == 64 ? 128 : N == 32 ? 192 : 256;
 }
 bool use_f32_chunks(int dtype, int64_t N, int64_t T, int64_t BH,
@@ -204,8 +217,10 @@ bool use_f32_chunks(int dtype, int64_t N, int64_t T, int64_t BH,
     if (N != 16 && N != 32 && N != 64 && N != 128) return false;
     if (dtype == RWKV7M_DTYPE_BF16 && N == 64) return false;
     if (token_stride * 64 >= (int64_t(1) << 31)) return false;
-    return T >= f32_min_tokens(backward, N) && BH <= (int64_t(1) << 22) &&
-           all_aligned16(ptrs);
+    if (BH > (int64_t(1) << 22) || !all_aligned16(ptrs)) return false;
+    const int cus = rwkv7m::device_cus();
+    if (!backward && N <= 64 && BH > cus) return false;
+    return T >= f32_min_tokens(backward, N, BH > cus / 4);
 }
 
 int forward_impl(const char* fn, int dtype, int64_t T, int64_t B, int64_t H,

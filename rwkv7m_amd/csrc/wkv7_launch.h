@@ -118,6 +118,9 @@ void set_backward_segments(int k);
 
 hipError_t launch_seq_forward(const SeqFwdArgs& p, hipStream_t stream);
 
+// CUs of the current device.
+int device_cus();
+
 // Chunked fp32 kernels (wkv7_f32.hip) for the calls the sequential ones
 // served: N in {16, 32, 64, 128} (64 with fp32 vectors only), 16-byte aligned
 // buffers, fp32 checkpoints every multiple of 16 tokens (backward: every

@@ -867,6 +867,8 @@ void set_forward_segments(int k) {
     g_force_fwd_segments.store(k < 0 ? 0 : k, std::memory_order_relaxed);
 }
 
+int device_cus() { return fwd_cu_count(); }
+
 hipError_t launch_wave_forward(const ChunkFwdArgs& p, hipStream_t stream) {
     // p.L: the checkpoint interval, a multiple of the 16-token chunk
     if (p.L % WL != 0 || p.L / WL < 1 || p.L / WL > 4)

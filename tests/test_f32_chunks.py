@@ -225,11 +225,12 @@ def test_segment_of_one_partial_chunk(hip):
 
 
 @pytest.mark.parametrize("N,dtype,B,H,T", [(128, torch.bfloat16, 32, 32, 181),
-                                           (64, torch.float32, 30, 100, 150)])
+                                           (64, torch.float32, 8, 32, 1366)])
 def test_time_segments(hip, N, dtype, B, H, T):
-    """Many heads: the workspace holds four chunks (N = 128, interval 32) or
-    three (N = 64) of 16 tokens forward and one backward, so the state, its
-    cotangent and the checkpoints pass from segment to segment.  Heads equal
+    """Many heads: the workspace holds five chunks of 16 tokens forward (four at
+    interval 32) and one backward at N = 128, 39 (38) and 19 at N = 64, so the
+    state, its cotangent and the checkpoints pass from segment to segment,
+    three times and more.  Heads equal
     the same heads in a call of few (one segment) bit for bit; three heads have
     a chunk out of range, in the first, a middle and the last segment."""
     tag = f"T{T} B{B} H{H} N{N} {dtype}"
@@ -290,3 +291,59 @@ def test_time_segments(hip, N, dtype, B, H, T):
     # (the last entry is the final state)
     eck = np.concatenate([eck[:-1:2], eck[-1:]])
     _close("ckpt", big[32]["ckpt"], eck, 1e-4, tag + " interval 32")
+
+
+@pytest.mark.parametrize("N,dtype", [(16, torch.bfloat16), (32, torch.float32),
+                                     (64, torch.float32)])
+def test_forward_of_more_heads_than_cus(hip, N, dtype):
+    """Up to a head a CU the chunked forward, past that the sequential one;
+    the backward is chunked either way, from either's checkpoints."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    T = 336
+    for H, path in ((cus, "f32_forward"), (cus + 1, "seq_forward")):
+        print("case: fp32 dispatch by heads", N, H, flush=True)
+        inp = make_inputs(T, 1, H, N, dtype=dtype, seed=4, state_std=0.1,
+                          dstate_std=0.1)
+        d = _dev(inp, "tbhn")
+        vecs = [d[n] for n in (*NAMES, "s0")]
+        hip.forward(*vecs)
+        assert hip.last_path() == path
+        (y, s_t), aux = hip.forward_with_aux(*vecs)
+        assert hip.last_path() == path
+        g = hip.backward(*vecs, d["dy"], d["ds_t"], *aux)
+        assert hip.last_path() == "f32_backward"
+        pick = slice(H - 2, H)
+        host = [_np(inp[n][:, :, pick]) for n in NAMES]
+        host.append(_np(inp["s0"][:, pick]))
+        ey, es = oracle.forward(*host)
+        eg = oracle.backward(*host, _np(inp["dy"][:, :, pick]),
+                             _np(inp["ds_t"][:, pick]))
+        _close("y", y[:, :, pick], ey, TOL[dtype], path)
+        _close("s_t", s_t[:, pick], es, 1e-4, path)
+        for n, a, e in zip(GRADS, g, eg):
+            a = a[:, pick] if n == "ds0" else a[:, :, pick]
+            _close(n, a, e, 1e-4 if n == "ds0" else TOL[dtype], path)
+
+
+@pytest.mark.parametrize("N,few,many", [(16, 256, 320), (32, 192, 320),
+                                        (64, 128, 192), (128, 64, 96)])
+def test_forward_dispatch_by_tokens(hip, N, few, many):
+    """The forward's shortest chunked calls, to a quarter of the CUs in heads
+    and past it; both kernels give the same heads the same results."""
+    q = torch.cuda.get_device_properties(0).multi_processor_count // 4
+    print("case: fp32 dispatch by tokens", N, flush=True)
+    for T in (few - 1, few, many - 1, many):
+        inp = make_inputs(T, 1, q + 1, N, dtype=torch.float32, seed=T,
+                          state_std=0.1, device="cuda", generator="torch")
+        vecs = [inp[n] for n in (*NAMES, "s0")]
+        outs = []
+        for H, line in ((q, few), (q + 1, many)):
+            y, s_t = hip.forward(*(x[:, :, :H].contiguous()
+                                   for x in vecs[:6]),
+                                 vecs[6][:, :H].contiguous())
+            assert hip.last_path() == ("f32_forward" if T >= line else
+                                       "seq_forward"), (T, H)
+            outs.append((y[:, :, :q], s_t[:, :q]))
+        torch.cuda.synchronize()
+        for a, b in zip(*outs):  # (2e-6: the kernels' own errors, twice)
+            assert float((a - b).norm() / b.norm()) <= 2e-6
