@@ -447,8 +447,8 @@ __device__ __forceinline__ d4 inverse(d4 a, d4 at, int l) {
 
 // One workgroup per chunk and head: bound by the inverse's products on one
 // wave, ten in float64 of which four follow each other, hidden by the other
-// chunks' workgroups on the CU (24 KB of LDS each at N = 64).  96 heads of 64,
-// 32 chunks: forward 40, backward 50 us (all float32: 31 and 43).
+// chunks' workgroups on the CU (22 and 28 KB of LDS each at N = 64).  96 heads
+// of 64, 32 chunks: forward 40, backward 50 us (all float32: 31 and 43).
 template <int N, typename VT, bool BWD>
 __global__ void __launch_bounds__(256, 2) f32_prep_kernel(Args A) {
     using W = Ws<N, BWD>;

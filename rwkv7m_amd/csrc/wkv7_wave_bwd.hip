@@ -679,35 +679,20 @@ __device__ __forceinline__ void work(const BwdArgs& A, int w, int lane0) {
                 pk8(as_i16x4(raw[6][2 * kp]), as_i16x4(raw[6][2 * kp + 1]));
         }
 
-        // ---- the 16 x 16 matrices (K = 64) ---------------------------------
-        f32x4_t mA = zero4(), mAT = zero4(), mAak = zero4(), mAakT = zero4(),
-                mArb = zero4(), mArbT = zero4(), mArk = zero4();
+        // ---- Aab (K = 64) --------------------------------------------------
+        // (its inverse before the other matrices: the choice of its products
+        // is a branch, and with the others live across it the summing
+        // instances spilled 38 to 47 registers, 20 % slower at L = 32)
+        f32x4_t mA = zero4(), mAT = zero4();
 #pragma unroll
         for (int kp = 0; kp < 2; ++kp) {
             const bf16x8_t a8 = pk8(tA[2 * kp], tA[2 * kp + 1]);
             const bf16x8_t b8 = pk8(tB[2 * kp], tB[2 * kp + 1]);
-            const bf16x8_t k8 = pk8(tK[2 * kp], tK[2 * kp + 1]);
-            const bf16x8_t r8 = pk8(tR[2 * kp], tR[2 * kp + 1]);
-            mfma(mA, a8, b8);     // Aab[t][s] = A~_t . B~_s
-            mfma(mAT, b8, a8);    // Aab^T
-            mfma(mAak, a8, k8);   // Aak[t][s] = A~_t . K~_s
-            mfma(mAakT, k8, a8);  // Aak^T
-            mfma(mArb, r8, b8);   // Arb[t][s] = R~_t . B~_s
-            mfma(mArbT, b8, r8);  // Arb^T
-            mfma(mArk, r8, k8);   // Ark[t][s] = R~_t . K~_s
+            mfma(mA, a8, b8);   // Aab[t][s] = A~_t . B~_s
+            mfma(mAT, b8, a8);  // Aab^T
         }
-        mA = mask4(mA, lr, lq, true, true);          // s < t
+        mA = mask4(mA, lr, lq, true, true);  // s < t
         mAT = mask4(mAT, lr, lq, true, false);
-        mAak = mask4(mAak, lr, lq, true, true);
-        mAakT = mask4(mAakT, lr, lq, true, false);
-        mArb = mask4(mArb, lr, lq, false, true);     // s <= t
-        mArbT = mask4(mArbT, lr, lq, false, false);
-        mArk = mask4(mArk, lr, lq, false, true);
-        const i16x4_t kAakA = kq(mAakT);  // A operand: Aak
-        const i16x4_t kAakB = kq(mAak);   // B operand: Aak
-        const i16x4_t kArbTA = kq(mArb);  // A operand: Arb^T
-        const i16x4_t kArbA = kq(mArbT);  // A operand: Arb
-        const i16x4_t kArkB = kq(mArk);   // B operand: Ark
 
         // ---- Minv = (I - Aab)^{-1} = (I + A)(I + A^2)(I + A^4)(I + A^8) ----
         // kMinv = kq(D(Minv^T)): A operand Minv, B operand Minv^T;
@@ -738,11 +723,41 @@ __device__ __forceinline__ void work(const BwdArgs& A, int w, int lane0) {
             mfma16(x8, pt4, px4);    // A^8
             const i16x4_t pq2t = kq(q2t), px8 = kq(x8);
             f32x4_t dM = q2, dMT = q2t;
-            mfma16(dM, pq2t, px8);   // Minv = Q2 + Q2 A^8
-            mfma16(dMT, px8, pq2t);  // Minv^T = Q2^T + (A^8)^T Q2^T
+            if (__builtin_expect(large_powers(x4), 0)) {
+                inverse32<true>(mA, mAT, lr, lq, dM, dMT);
+            } else {
+                mfma16(dM, pq2t, px8);   // Minv = Q2 + Q2 A^8
+                mfma16(dMT, px8, pq2t);  // Minv^T = Q2^T + (A^8)^T Q2^T
+            }
             kMinv = kq(dMT);
             kMinvT = kq(dM);
         }
+
+        // ---- the other 16 x 16 matrices (K = 64) ---------------------------
+        f32x4_t mAak = zero4(), mAakT = zero4(), mArb = zero4(),
+                mArbT = zero4(), mArk = zero4();
+#pragma unroll
+        for (int kp = 0; kp < 2; ++kp) {
+            const bf16x8_t a8 = pk8(tA[2 * kp], tA[2 * kp + 1]);
+            const bf16x8_t b8 = pk8(tB[2 * kp], tB[2 * kp + 1]);
+            const bf16x8_t k8 = pk8(tK[2 * kp], tK[2 * kp + 1]);
+            const bf16x8_t r8 = pk8(tR[2 * kp], tR[2 * kp + 1]);
+            mfma(mAak, a8, k8);   // Aak[t][s] = A~_t . K~_s
+            mfma(mAakT, k8, a8);  // Aak^T
+            mfma(mArb, r8, b8);   // Arb[t][s] = R~_t . B~_s
+            mfma(mArbT, b8, r8);  // Arb^T
+            mfma(mArk, r8, k8);   // Ark[t][s] = R~_t . K~_s
+        }
+        mAak = mask4(mAak, lr, lq, true, true);
+        mAakT = mask4(mAakT, lr, lq, true, false);
+        mArb = mask4(mArb, lr, lq, false, true);     // s <= t
+        mArbT = mask4(mArbT, lr, lq, false, false);
+        mArk = mask4(mArk, lr, lq, false, true);
+        const i16x4_t kAakA = kq(mAakT);  // A operand: Aak
+        const i16x4_t kAakB = kq(mAak);   // B operand: Aak
+        const i16x4_t kArbTA = kq(mArb);  // A operand: Arb^T
+        const i16x4_t kArbA = kq(mArbT);  // A operand: Arb
+        const i16x4_t kArkB = kq(mArk);   // B operand: Ark
 
         // The phases after the factors, as calls: the map (the chains'
         // operands), U and X (need S_0), and dX, dU, dV (need D).  At an

@@ -99,6 +99,59 @@ __device__ __forceinline__ void mfma(f32x4_t& acc, const bf16x8_t& a,
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
 }
 
+// D(M Y) + c from D(M^T) and D(Y), in float32 (four v_mfma_f32_16x16x4_f32).
+__device__ __forceinline__ f32x4_t mm32(const f32x4_t& mt, const f32x4_t& y,
+                                        f32x4_t c = {0.f, 0.f, 0.f, 0.f}) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(mt[e], y[e], c, 0, 0, 0);
+    return c;
+}
+
+// The inverse of I - A, A = Aab strictly lower, is formed as (I + A)(I + A^2)
+// (I + A^4)(I + A^8) with bf16 operands.  Keys that resemble each other in a
+// chunk (repeated tokens) under slow decay put A near -a below the diagonal:
+// its powers grow to 1e3 and cancel, and their rounding, 2^-9 of the largest,
+// stays: y was 1 % off where they reach 10, 10 % at 100, and from 500 on the
+// next chunks amplified it without bound.  A chunk with an entry of A^4 above
+// this takes the products in float32 instead: y is 0.4 to 1 % off on all of
+// these, and a step of such chunks alone takes 13 % longer (256 heads of 512
+// tokens: forward 43 -> 48 us, backward 76 -> 86).  At independent keys the
+// entries are about 0.01, so such chunks keep their bits, and the choice costs
+// up to 1 % (2 x 1999 tokens of 32 heads: forward 93.4 -> 93.9 us; at interval
+// 32 the backward 262 -> 266; a step of 8 x 4096 tokens 828 -> 827).
+constexpr float kMaxPower = 1.f;
+__device__ __forceinline__ bool large_powers(const f32x4_t& x4) {
+    const float m = fmaxf(fmaxf(fabsf(x4[0]), fabsf(x4[1])),
+                          fmaxf(fabsf(x4[2]), fabsf(x4[3])));
+    return __builtin_amdgcn_ballot_w64(m > kMaxPower) != 0;
+}
+
+// D(Minv^T), and D(Minv) where wanted, from D(A) and D(A^T); r = lane % 16,
+// q = lane / 16.
+template <bool BOTH>
+__device__ __forceinline__ void inverse32(const f32x4_t& a, const f32x4_t& at,
+                                          int r, int q, f32x4_t& m,
+                                          f32x4_t& mt) {
+    const f32x4_t a2 = mm32(at, a), a2t = mm32(a, at);
+    f32x4_t q1 = a + a2, q1t = at + a2t;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float one = (4 * q + e == r) ? 1.f : 0.f;
+        q1[e] += one;
+        q1t[e] += one;
+    }
+    q1t = mm32(a2, at, q1t);
+    const f32x4_t a4 = mm32(a2t, a2), a4t = mm32(a2, a2t);
+    const f32x4_t a8 = mm32(a4t, a4);
+    const f32x4_t q2t = mm32(a4, q1t, q1t);
+    if constexpr (BOTH) {
+        q1 = mm32(at, a2, q1);
+        m = mm32(q2t, a8, mm32(q1t, a4, q1));
+    }
+    mt = mm32(a8, q2t, q2t);
+}
+
 // The chunk kernels' input vectors.  Pointers are picked by a switch over
 // kernel arguments (never from an indexed array) so that the compiler keeps
 // them in the global address space: flat loads would also count against the

@@ -364,8 +364,12 @@ __device__ __forceinline__ void produce(const FwdArgs& A, WaveFwdSmem& sm,
             f32x4_t q2t = q1t, x8 = zero4();
             mfma16(q2t, px4, pq1t);  // (Q1 + Q1 A^4)^T
             mfma16(x8, pt4, px4);    // A^8
-            dMT = q2t;
-            mfma16(dMT, kq(x8), kq(q2t));  // Minv^T = (Q2 + Q2 A^8)^T
+            if (__builtin_expect(large_powers(x4), 0)) {
+                inverse32<false>(mA, mAT, lr, lq, dMT, dMT);
+            } else {
+                dMT = q2t;
+                mfma16(dMT, kq(x8), kq(q2t));  // Minv^T = (Q2 + Q2 A^8)^T
+            }
         }
 
         // ---- products over the chunk (K = 16) ------------------------------
